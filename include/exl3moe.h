@@ -99,9 +99,9 @@ int exl3_set_decision_log(int32_t* buf, int64_t cap_words);
 
 /* ---- routed-expert MoE --------------------------------------------------------------------------------------------- */
 
-/* workspace bytes of an exl3_moe_forward call with these sizes (decode kernels for M < prefill_min_m: the blob
- * pointer of every pick; the prefill path otherwise: sorted routing, input Hadamards [M topk][2][H] fp16, abuf
- * [M topk][I] fp16, y [M topk][H] fp16). The decode kernel's cross-workgroup exchange is not in the workspace: the
+/* workspace bytes of an exl3_moe_forward call with these sizes (small decode calls: the blob pointer of every pick; the
+ * grouped kernels otherwise: sorted routing, input Hadamards [M topk][2][H] fp16, abuf [M topk][I] fp16, y [M topk][H]
+ * fp16, or fp32 below prefill_min_m; calls of more picks than one pass takes share the workspace of a pass). The decode kernel's cross-workgroup exchange is not in the workspace: the
  * library owns one zeroed device buffer per device and grows it when a call needs more (hipMalloc + hipMemset, after
  * a device synchronisation; the replaced buffer stays allocated, since graphs captured earlier still address it); a
  * call that would grow it while its stream is being captured fails with EXL3_EUNSUPPORTED, so run one call of the
@@ -110,9 +110,10 @@ size_t exl3_moe_forward_workspace(int M, int H, int I, int topk, int n_experts);
 
 /* moe_forward (a8:1221-1225 -> moe_forward_impl a8:1263-1314): out[m] = sum_k w[m,k] * expert(ids[m,k])(x[m]).
  * x, out: [M, H] with row strides, dtype EXL3_DT_*; ids int32 / w fp32 [M, topk] contiguous; ptrs int64 [n_experts]
- * blob addresses (device slots or device-mapped pinned host memory). M < prefill_min_m runs the fused decode kernel
- * (M <= 256 rows, M * topk <= 1024 pairs); M >= prefill_min_m the prefill path (moe_prefill a8:792-828): token sort,
- * grouped MFMA GEMMs with the trellis decoded into LDS, y in fp16, combine (needs H % 256 == 0). */
+ * blob addresses (device slots or device-mapped pinned host memory). Small decode calls run the fused decode kernel;
+ * with H % 256 == 0, decode calls from topk * M * I = 60,000 on and every call of M >= prefill_min_m (or of more than
+ * 1024 picks or 256 rows, which need it) run the grouped kernels (moe_prefill a8:792-828): token sort, the experts'
+ * trellis decoded into MFMA registers once for all their rows, combine; y in fp16 from prefill_min_m on. */
 int exl3_moe_forward(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
                      const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
                      int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream);
@@ -131,9 +132,9 @@ int exl3_moe_forward_cached(const void* x, int x_dtype, int64_t x_stride, int M,
 /* The same call without any allocation (no reference counterpart: the reference always passes a workspace that
  * torch allocates, a8:1229-1261). For callers that cannot allocate device memory: code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc. The decode scratch (the blob pointer of every pick and the
- * cross-workgroup exchange words) comes from one static device array of EXL3_STATIC_SCRATCH_BYTES per device, held
- * until the process ends; its address is looked up on the first call on a device and the array is cleared then (one
- * fill kernel on `stream`). Limit: calls whose scratch exceeds the array (8 MiB: config-0 shapes up to 25 rows x
+ * cross-workgroup exchange words, or the grouped kernels' workspace) comes from two static device arrays of
+ * EXL3_STATIC_SCRATCH_BYTES (and 64 KiB) per device, held until the process ends; their addresses are looked up on
+ * the first call on a device and the exchange words cleared then (one fill kernel on `stream`). Limit: calls whose scratch exceeds the array (8 MiB: config-0 shapes up to 25 rows x
  * top-10, config-4 shapes up to 7 rows x top-8) and calls that would take the uncached path (M >= prefill_min_m, or
  * n_slots == 0) fail with EXL3_EUNSUPPORTED before anything is enqueued. Every call on one device shares the array
  * and it keeps the last call's contents: calls that overlap on one device (other streams) race; stream-ordered calls

@@ -89,21 +89,21 @@ struct DecodeArgs {
 struct AlignOut {
     int* act_expert; int* act_start; int* act_cnt; int* act_pstart; int* n_act;   // [A], [A], [A], [A], [1]
     int* pair_tok; int* pair_of; float* pair_w;                                    // [npairs] each
-    int* pair_exp;                                                                  // expert of each sorted pair or null
-    // the active experts again in GEMM dispatch order (descending 32-row block count, ties by ascending id), or null
-    int* ord_expert; int* ord_start; int* ord_cnt;                                  // [A] each
 };
 
-struct PrefillArgs {
+// picks grouped by expert, few rows each (moe_grouped.hip)
+struct GroupedArgs {
     const void* x; int x_dt; int64_t x_stride;     // activations [M, H]
     const int32_t* ids; const float* w;            // [M * topk]
-    int M, topk, npairs;
+    int M, topk, npairs, E;
     const int64_t* ptrs;                           // per-layer blob pointer table [E]
-    const int* ord_expert; const int* ord_start; const int* ord_cnt; const int* n_act;   // GEMM dispatch order
-    const int* pair_tok; const float* pair_w; const int* pair_of; const int* pair_exp;
-    _Float16* xh;                                  // [npairs (sorted)][2][H] input Hadamards (gate, up)
-    _Float16* abuf;                                // [npairs (sorted)][I]
-    _Float16* y;                                   // [npairs (sorted)][H], routing weight applied
+    int* perm;                                     // pick at every sorted position [npairs]
+    int rmax;                                      // rows of an item at most (64 or 192)
+    int* it_expert; int* it_start; int* it_cnt;    // items: up to rmax sorted positions of one expert, longest first
+    int* n_items;                                  // [2] items, and those of more than 16 rows (the first ones)
+    _Float16* xh;                                  // [npairs][2][H] input Hadamards (gate, up)
+    _Float16* abuf;                                // [npairs][I]
+    void* y;                                       // [npairs][H] fp32 or fp16, routing weight applied
     void* out; int64_t out_stride;                 // [M, H], dtype of x
     BlobGeom g;
 };
@@ -184,8 +184,10 @@ hipError_t launch_tier_exchange(uint8_t* flags, int64_t n_flags, const int32_t* 
 hipError_t launch_align(const int32_t* ids, const float* w, int npairs, int topk, int E, int pad, int* chunk_scratch,
                         const AlignOut& o, hipStream_t s);
 size_t align_scratch_bytes(int npairs, int E);
-size_t prefill_workspace_bytes(int M, int H, int I, int topk, int E);
-hipError_t launch_prefill(PrefillArgs a, int E, void* ws, hipStream_t s);
+
+// grouped.hip: y32 keeps the picks' outputs in fp32 (the decode sizes), else fp16 (as the prefill kernels do)
+size_t grouped_workspace_bytes(int M, int topk, int H, int I, int E, bool y32);
+hipError_t launch_grouped(const GroupedArgs& a, bool y32, void* ws, hipStream_t s);
 
 // 1024-row slices of H of the decode gate/up workgroups (one 128-row block per wave; H is a multiple of 128)
 __host__ __device__ static inline int gu_kslices(int H) { return (H + 1023) / 1024; }

@@ -258,10 +258,23 @@ int exl3_set_decision_log(int32_t* buf, int64_t cap_words) {
 static bool exceeds_decode(int M, int topk) { return (int64_t)M * topk > kMaxPairs || M > kMaxRows; }
 static bool use_prefill(int M, int topk) { return M >= g_cfg.prefill_min_m || exceeds_decode(M, topk); }
 
+// the grouped kernels (moe_grouped.hip) decode each expert's weights once for all of its picks, the fused decode kernel
+// once per pick: they take every call of the prefill sizes, and the decode sizes from picks * I = 60,000 on. Below it
+// the fused kernel's single launch is faster: at H 2048 / I 512, top-10, 54 us against 73 us for 8 rows of distinct
+// experts (80 picks) and 104 against 74 us for 16 Zipf rows; at H 4096 / I 1536, top-8, 66 against 85 us for 2 rows and
+// 184 against 151 us for 6.
+constexpr int64_t kGroupedMinWork = 60000;
+static bool use_grouped(int M, int topk, int H, int I) {
+    return H % 256 == 0 && (use_prefill(M, topk) || (int64_t)M * topk * I >= kGroupedMinWork);
+}
+// the picks' outputs stay fp32 at the decode sizes, and are fp16 at the prefill sizes (as the reference keeps them)
+static bool grouped_y32(int M, int topk) { return !use_prefill(M, topk); }
+
 size_t exl3_moe_forward_workspace(int M, int H, int I, int topk, int n_experts) {
     if (M <= 0 || topk <= 0 || H <= 0 || I <= 0) return 0;
     const int E = std::min(std::max(n_experts, 1), kMaxExperts);
-    return use_prefill(M, topk) ? prefill_workspace_bytes(M, H, I, topk, E) : decode_workspace_bytes(M * topk, H, I);
+    if (use_grouped(M, topk, H, I)) return grouped_workspace_bytes(M, topk, H, I, E, grouped_y32(M, topk));
+    return decode_workspace_bytes(M * topk, H, I);
 }
 
 static int64_t* pair_ptr_area(void* ws, int npairs, int H, int I) {
@@ -326,24 +339,27 @@ static int forward_impl(const void* x, int x_dtype, int64_t x_stride, int M, int
     if (!fill && use_prefill(M, topk)) {
         if (H % 256) return fail(EXL3_EUNSUPPORTED, "moe prefill: H %% 256 == 0 required (H=%d)", H);
         if ((int64_t)M * topk > (1 << 28)) return fail(EXL3_EUNSUPPORTED, "moe prefill: %d x %d pairs", M, topk);
-        const size_t need = prefill_workspace_bytes(M, H, I, topk, E);
+    }
+    if (!fill && use_grouped(M, topk, H, I)) {
+        const bool y32 = grouped_y32(M, topk);
+        const size_t need = grouped_workspace_bytes(M, topk, H, I, E, y32);
         if (!ws || ws_bytes < need)
-            return fail(EXL3_EWORKSPACE, "moe_forward (prefill): workspace %zu < %zu bytes", ws_bytes, need);
-        PrefillArgs pa{};
-        pa.x = x;
-        pa.x_dt = x_dtype;
-        pa.x_stride = x_stride;
-        pa.ids = ids;
-        pa.w = w;
-        pa.M = M;
-        pa.topk = topk;
-        pa.npairs = M * topk;
-        pa.ptrs = ptrs;
-        pa.out = out;
-        pa.out_stride = out_stride;
-        pa.g = blob_geom(H, I, K);
-        hipError_t e = launch_prefill(pa, E, ws, st);
-        return e == hipSuccess ? EXL3_OK : hip_fail(e, "moe prefill launch");
+            return fail(EXL3_EWORKSPACE, "moe_forward (grouped): workspace %zu < %zu bytes", ws_bytes, need);
+        GroupedArgs ga{};
+        ga.x = x;
+        ga.x_dt = x_dtype;
+        ga.x_stride = x_stride;
+        ga.ids = ids;
+        ga.w = w;
+        ga.M = M;
+        ga.topk = topk;
+        ga.E = E;
+        ga.ptrs = ptrs;
+        ga.out = out;
+        ga.out_stride = out_stride;
+        ga.g = blob_geom(H, I, K);
+        const hipError_t e = launch_grouped(ga, y32, ws, st);
+        return e == hipSuccess ? EXL3_OK : hip_fail(e, "moe grouped launch");
     }
     const int npairs = M * topk;
     if (npairs > kMaxPairs || M > kMaxRows)
@@ -595,6 +611,7 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
         return fail(EXL3_EINVAL, "moe_forward_cached: null cache state");
     const BlobGeom g = blob_geom(H, I, K);
     const int P = M * topk;
+    const bool grouped = exceeds_decode(M, topk) || use_grouped(M, topk, H, I);
     if (exceeds_decode(M, topk) && xb)
         return fail(EXL3_EUNSUPPORTED, "moe_forward_cached_static: %d x %d picks take the prefill kernels, which need "
                     "a workspace (use exl3_moe_forward_cached)", M, topk);
@@ -648,11 +665,11 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
     uint8_t* vict_res = ea.vr_meta ? nullptr : g_cfg.ram_res;
     ea.log = g_cfg.log;
     ea.log_cap = g_cfg.log_cap;
-    if (exceeds_decode(M, topk)) {
-        // more picks than the decode kernel takes: one ensure over all of them, victim write-back, fill copies and
-        // the commit, then the prefill kernels over the committed table (the caller's ids and w carry the tier mask)
+    if (grouped) {
+        // one ensure over all the picks, victim write-back, fill copies and the commit, then the grouped kernels over
+        // the committed table (the caller's ids and w carry the tier mask)
         if (H % 256) return fail(EXL3_EUNSUPPORTED, "moe_forward_cached: %d picks need the prefill kernels (H %% 256)", P);
-        const size_t need = prefill_workspace_bytes(M, H, I, topk, E);
+        const size_t need = grouped_workspace_bytes(M, topk, H, I, E, grouped_y32(M, topk));
         if (!workspace || workspace_bytes < need)
             return fail(EXL3_EWORKSPACE, "moe_forward_cached: workspace %zu < %zu bytes", workspace_bytes, need);
         ea.pend = g_cfg.n_layers > 0 ? g_cfg.pend : nullptr;   // commit finished copy-engine plans first
@@ -720,8 +737,13 @@ static_assert(decode_workspace_bytes(kMaxPairs, 0, 0) <= kStaticPtrBytes,
               "the pointer area of the static scratch must hold the workspace of the largest decode call");
 static_assert(kStaticPtrBytes % 256 == 0 && kStaticPtrBytes < kStaticScratchBytes, "static scratch layout");
 static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
+// the grouped kernels' workspace of a static call, in an array of its own (its data could pass as a tag): per pick it
+// takes 8 H + 2 I bytes where the exchange words take at least 16 I + 8 H, so every call that the exchange words admit
+// fits beside the sort's lists
+constexpr size_t kStaticGroupedBytes = kStaticScratchBytes + (64 << 10);
+static __device__ __align__(256) uint8_t grouped_scratch[kStaticGroupedBytes];
 static std::mutex g_scratch_mu;
-static uint8_t* g_scratch_ptr[kMaxDevices];
+static uint8_t* g_scratch_ptr[kMaxDevices][2];
 
 __global__ void zero_fill_kernel(uint4* p, size_t n16) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x)
@@ -730,21 +752,25 @@ __global__ void zero_fill_kernel(uint4* p, size_t n16) {
 
 // this device's scratch, set up on first use: its address, then one clear by a kernel on `st` (no memset node if the
 // first call is being captured; the exchange words only need to carry no live tag, which zero never is)
-static int static_scratch(hipStream_t st, uint8_t** out) {
+static int static_scratch(hipStream_t st, uint8_t** out, uint8_t** grouped) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     if (dev < 0 || dev >= kMaxDevices) return fail(EXL3_EUNSUPPORTED, "device %d >= %d", dev, kMaxDevices);
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_ptr[dev]) {
+    if (!g_scratch_ptr[dev][0]) {
         void* p = nullptr;
+        void* q = nullptr;
         e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p) return hip_fail(e, "static scratch: hipGetSymbolAddress");
+        if (e == hipSuccess) e = hipGetSymbolAddress(&q, HIP_SYMBOL(grouped_scratch));
+        if (e != hipSuccess || !p || !q) return hip_fail(e, "static scratch: hipGetSymbolAddress");
         hipLaunchKernelGGL(zero_fill_kernel, dim3(256), dim3(256), 0, st, (uint4*)p, kStaticScratchBytes / 16);
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "static scratch: clear");
-        g_scratch_ptr[dev] = (uint8_t*)p;
+        g_scratch_ptr[dev][1] = (uint8_t*)q;
+        g_scratch_ptr[dev][0] = (uint8_t*)p;
     }
-    *out = g_scratch_ptr[dev];
+    *out = g_scratch_ptr[dev][0];
+    *grouped = g_scratch_ptr[dev][1];
     return EXL3_OK;
 }
 
@@ -780,11 +806,14 @@ int exl3_moe_forward_cached_static(const void* x, int x_dtype, int64_t x_stride,
         return fail(EXL3_EUNSUPPORTED, "moe_forward_cached_static: the call needs %zu bytes of scratch, the static "
                     "scratch holds %zu (fewer rows, or exl3_moe_forward_cached)", need, kStaticScratchBytes);
     uint8_t* sp = nullptr;
-    const int r = static_scratch((hipStream_t)stream, &sp);
+    uint8_t* gp = nullptr;
+    const int r = static_scratch((hipStream_t)stream, &sp, &gp);
     if (r) return r;
+    const bool grouped = !exceeds_decode(M, topk) && use_grouped(M, topk, H, I);
     return cached_impl(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs_all, layer, slot_of, slot_key,
                        slot_last, tick, n_slots, host_base, slot_base, fill_all, fill_list, max_fill, I, K, n_experts,
-                       out, out_stride, sp, ws, stream, (uint64_t*)(sp + kStaticPtrBytes));
+                       out, out_stride, grouped ? gp : sp, grouped ? kStaticGroupedBytes : ws, stream,
+                       (uint64_t*)(sp + kStaticPtrBytes));
 }
 
 size_t exl3_moe_align_workspace(int M, int topk, int n_experts) {
@@ -811,7 +840,6 @@ int exl3_moe_align(const int32_t* topk_ids, const float* topk_w, int M, int topk
     o.pair_tok = ib + 4 * A + 1;
     o.pair_of = o.pair_tok + npairs;
     o.pair_w = fb;
-    o.pair_exp = nullptr;
     hipError_t e = launch_align(topk_ids, topk_w, npairs, topk, n_experts, pad, (int*)workspace, o, (hipStream_t)stream);
     return e == hipSuccess ? EXL3_OK : hip_fail(e, "moe_align launch");
 }
