@@ -264,6 +264,15 @@ size_t exl3_linear_workspace(int M, int k, int n);
 int exl3_linear_small(const void* x, int x_dtype, int64_t x_stride, int M, int k, int n, const void* trellis, int K,
                       int cb, const void* suh, int S, const void* svh, const int32_t* shard_of_nb, void* out,
                       int out_dtype, int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same linear for any number of rows, with the input Hadamards, the trellis decode and the products in kernels of
+ * its own (exl3_ops.sycl:651-757, the path above the fused rows). group_bounds: host [S + 1], shard g's columns
+ * [group_bounds[g], group_bounds[g + 1]), multiples of width (256 or 128). S at most 16. The workspace (device, exl3_linear_rows_workspace bytes, no state between calls) holds the input
+ * Hadamards and the partial sums. EXL3_EUNSUPPORTED if S M k fp16 values or the trellis reach 2 GiB. */
+size_t exl3_linear_rows_workspace(int M, int k, int n, int S, int width);
+int exl3_linear_rows(const void* x, int x_dtype, int64_t x_stride, int M, int k, int n, const void* trellis, int K,
+                     int cb, const void* suh, int S, const void* svh, const int64_t* group_bounds, int width, void* out,
+                     int out_dtype, int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream);
 /* exl3_had_in_rm (exl3_ops.sycl:602-608): xh fp16 [S][M][k] = fp16(H(fp16(x * suh[g])) / sqrt 128) */
 int exl3_had_in(const void* x, int x_dtype, int64_t x_stride, int M, int k, const void* suh, int S, void* xh,
                 void* stream);

@@ -20,7 +20,9 @@ BUILD = os.path.join(HERE, "_build")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["moe_decode.hip", "moe_cache.hip", "moe_align.hip", "moe_grouped.hip", "linear.hip", "moe_capi.hip"]
+HIP_SOURCES = ["moe_products_k3.hip", "moe_products_k2.hip", "moe_products_k4.hip", "linear_rows_k4.hip",
+               "linear_rows_k23.hip", "linear_rows_k56.hip", "linear_rows_k6.hip", "moe_decode.hip", "linear.hip",
+               "moe_cache.hip", "moe_align.hip", "moe_grouped.hip", "linear_rows.hip", "moe_capi.hip"]
 HOST_SOURCES = ["tier_host.cpp"]          # host-only C++ (g++)
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
                "-packed-fp32-ops", "-Wno-unused-command-line-argument"]

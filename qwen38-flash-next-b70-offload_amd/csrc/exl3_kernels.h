@@ -112,6 +112,7 @@ constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // the dense EXL3 linear (linear.hip): out[M, n] = svh * H(sum_k xh[shard of n][m][k] W[k][n]) / sqrt 128
 constexpr int kLinMaxRows = 8;       // rows of the fused small-M path
+constexpr int kLinMaxGroups = 16;    // shards of a linear_rows call
 struct LinearArgs {
     const void* x; int x_dt; int64_t x_stride;     // activations [M, k]
     int M, k, n, S;                                // rows, input and output features, shards
@@ -119,6 +120,7 @@ struct LinearArgs {
     const _Float16* suh;                           // [S][k]
     const _Float16* svh;                           // [n]
     const int32_t* shard_of_nb;                    // [n/128]
+    int first[kLinMaxGroups];                      // linear_rows: every shard's first column
     _Float16* xh;                                  // [S][M][k] (the large-M path's input Hadamards)
     uint64_t* part;                                // [P][M][n] tagged partial sums over the K-slices: zero on
                                                    // entry, left zero
@@ -131,6 +133,16 @@ hipError_t launch_linear_had_in(const LinearArgs& a, hipStream_t s);
 // codebook cb: 2 mul1 (K = 2..6), 1 mcg or 0 3inst (K = 4, 6)
 hipError_t launch_linear_small(int K, int cb, const LinearArgs& a, void* out, int out_dt, int64_t out_stride,
                                hipStream_t s);
+// the linear for more rows (linear_rows.hip): xh [S][M][k] and part fp32 [P][M][n] (P > 1) are workspaces; every shard's
+// columns are a multiple of width (256 or 128); S M k and k n K / 8 bytes below 2 GiB
+// 16-row blocks of a workgroup: up to 64 rows in one tile, above that tiles of 128 (each tile decodes the weights again)
+static inline int linear_rows_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
+int linear_rows_slices(int M, int k, int n, int width);
+template <int K, int CB>
+void linear_rows_product(const LinearArgs& a, int width, float* part, void* out, int out_dt, int64_t out_stride,
+                         hipStream_t s);
+hipError_t launch_linear_rows(int K, int cb, const LinearArgs& a, int width, float* part, void* out, int out_dt,
+                              int64_t out_stride, hipStream_t s);
 // out = svh * H(sum of P parts) / sqrt 128; parts fp32 (y_half 0) or one fp16 matrix (y_half 1, P 1)
 hipError_t launch_linear_had_out(const void* parts, int y_half, int P, int M, int n, const _Float16* svh, void* out,
                                  int out_dt, int64_t out_stride, hipStream_t s);
@@ -186,6 +198,10 @@ hipError_t launch_align(const int32_t* ids, const float* w, int npairs, int topk
 size_t align_scratch_bytes(int npairs, int E);
 
 // grouped.hip: y32 keeps the picks' outputs in fp32 (the decode sizes), else fp16 (as the prefill kernels do)
+// an upper bound of a call's items: every expert's last one, and one more per 64 picks (items are cut at 64 rows or more)
+static inline size_t grouped_max_items(size_t np, int E) { return (np < (size_t)E ? np : (size_t)E) + np / 64; }
+// gate/up and down at bitrate K (moe_products.cuh)
+template <int K> void launch_products(const GroupedArgs& a, bool y32, hipStream_t s);
 size_t grouped_workspace_bytes(int M, int topk, int H, int I, int E, bool y32);
 hipError_t launch_grouped(const GroupedArgs& a, bool y32, void* ws, hipStream_t s);
 

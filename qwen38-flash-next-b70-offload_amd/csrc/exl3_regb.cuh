@@ -184,7 +184,9 @@ __device__ __forceinline__ uint32_t a_slot16(int r, int j) { return (uint32_t)(r
 
 // The same product with the A rows staged through LDS for the WV waves of a workgroup (64 columns each), for more rows:
 // NPROJ matrices of 16 NB rows (wave's matrix: proj), double-buffered, one barrier per chunk. Thread unit i covers 32
-// bytes of one row of one matrix: soff[i] its byte offset in ra (kOob reads zeros), written where unit_lds says.
+// bytes of one row of one matrix: soff[i] its byte offset in ra (kOob reads zeros). SD chunks of A are in flight in
+// registers ahead of their LDS stores. PF > 0: PF fragments of A are read ahead of their MFMAs, the first ones before the
+// chunk's decode (where the accumulators leave the registers for them).
 template <int NB, int WV, int NPROJ>
 struct AUnits {
     static constexpr int N = NPROJ * 16 * NB * 4;    // 32-byte units of a chunk
@@ -196,53 +198,56 @@ struct AUnits {
     static constexpr int kBuf = NPROJ * 16 * NB * 128;
 };
 
-template <int K, int NB, int WV, int NPROJ, bool NAT, int CB, typename R>
+template <int K, int NB, int WV, int NPROJ, bool NAT, int CB, int SD, int PF, typename R>
 __device__ __forceinline__ void regb_lds_core(R rw, uint32_t woff, int tiles_n, R ra,
                                               const uint32_t (&soff)[AUnits<NB, WV, NPROJ>::NU], int nch, int proj,
                                               uint8_t* lds, float4_t (&acc)[NB][2][2]) {
     using B = RegB<K, NAT, CB>;
     using U = AUnits<NB, WV, NPROJ>;
-    constexpr int PD = NB <= 4 ? 4 : 2;
+    constexpr int PD = NB <= 4 && B::NW <= 8 ? 4 : 2;
+    static_assert(PD % 2 == 0 && PD % SD == 0, "buffer and register indices are compile-time within PD chunks");
     const uint32_t cb = B::chunk_bytes(tiles_n);
     const int src = B::prev_lane(), l = lane_id(), q = l >> 4;
     uint32_t wd[PD][B::NW];
-    u32x4_t st[U::NU][2];
-    auto stage_load = [&](int c) {
+    u32x4_t st[SD][U::NU][2];
+    auto stage_load = [&](int s, int c) {        // (past the last chunk: the last one again)
 #pragma unroll
         for (int i = 0; i < U::NU; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                st[i][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(soff[i] + 16 * j),
-                                                                                            c * 128, 0));
+                st[s][i][j] = __builtin_bit_cast(
+                    u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(soff[i] + 16 * j), min(c, nch - 1) * 128, 0));
     };
-    auto stage_store = [&](int buf) {
+    auto stage_store = [&](int s, int buf) {
 #pragma unroll
         for (int i = 0; i < U::NU; ++i)
             if (U::live(i)) {
                 uint8_t* p = lds + buf * U::kBuf + U::proj(i) * (16 * NB * 128);
                 const int r = U::row(i), j = 2 * (U::index(i) & 3);
+                const u32x4_t lo = st[s][i][0], hi = st[s][i][1];
                 if constexpr (B::F8) {
-                    *(u32x4_t*)(p + a_slot16(r, j)) = st[i][0];
-                    *(u32x4_t*)(p + a_slot16(r, j + 1)) = st[i][1];
+                    *(u32x4_t*)(p + a_slot16(r, j)) = lo;
+                    *(u32x4_t*)(p + a_slot16(r, j + 1)) = hi;
                 } else {
-                    *(u32x4_t*)(p + a_slot16(r, j)) = u32x4_t{st[i][0][0], st[i][0][1], st[i][1][0], st[i][1][1]};
-                    *(u32x4_t*)(p + a_slot16(r, j + 1)) = u32x4_t{st[i][0][2], st[i][0][3], st[i][1][2], st[i][1][3]};
+                    *(u32x4_t*)(p + a_slot16(r, j)) = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+                    *(u32x4_t*)(p + a_slot16(r, j + 1)) = u32x4_t{lo[2], lo[3], hi[2], hi[3]};
                 }
             }
     };
-    stage_load(0);
+#pragma unroll
+    for (int j = 0; j < SD; ++j) stage_load(j, j);
 #pragma unroll
     for (int j = 0; j < PD; ++j) B::load(wd[j], rw, j < nch ? woff + (uint32_t)j * cb : kOob, tiles_n);
-    stage_store(0);
-    stage_load(min(1, nch - 1));
+    stage_store(0, 0);
+    stage_load(0, SD);
     __syncthreads();
     const uint8_t* ab = lds + proj * (16 * NB * 128);
     for (int c = 0; c < nch; c += PD) {
 #pragma unroll
         for (int j = 0; j < PD; ++j) {
             if (c + j >= nch) break;
-            if (c + j + 1 < nch) stage_store((j + 1) & 1);
-            stage_load(min(c + j + 2, nch - 1));
+            if (c + j + 1 < nch) stage_store((j + 1) % SD, (j + 1) & 1);
+            stage_load((j + 1) % SD, c + j + 1 + SD);
             const uint8_t* a0 = ab + (j & 1) * U::kBuf;
             typename B::Dec d[2];
             auto half = [&](auto F) {
@@ -251,21 +256,32 @@ __device__ __forceinline__ void regb_lds_core(R rw, uint32_t woff, int tiles_n, 
                     B::prep(d[0], wd[j], B::F8 ? 0 : f, 0, src);
                     B::prep(d[1], wd[j], B::F8 ? 0 : f, 1, src);
                 }
-                half8_t w[2][2];
+                const uint8_t* af = a0 + a_slot16(l & 15, B::F8 ? 2 * q + f : 4 * f + q);
+                auto rd = [&](int b) { return *(const half8_t*)(af + b * 16 * 128); };
+                half8_t w[2][2], a[PF > 0 ? PF : 1];
+                if constexpr (PF > 0) {          // before the decode, so that it covers their latency
+#pragma unroll
+                    for (int b = 0; b < PF; ++b) a[b] = rd(b);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
 #pragma unroll
                 for (int cc = 0; cc < 2; ++cc) {
                     w[cc][0] = B::template frag<f, 0>(d[cc]);
                     w[cc][1] = B::template frag<f, 1>(d[cc]);
                 }
-                const uint8_t* af = a0 + a_slot16(l & 15, B::F8 ? 2 * q + f : 4 * f + q);
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const half8_t a = *(const half8_t*)(af + b * 16 * 128);
+                    const half8_t ab16 = PF > 0 ? a[PF > 0 ? b % PF : 0] : rd(b);
 #pragma unroll
                     for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
-                            acc[b][cc][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, w[cc][h], acc[b][cc][h], 0, 0, 0);
+                            acc[b][cc][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ab16, w[cc][h], acc[b][cc][h], 0, 0, 0);
+                    if (PF > 0 && b + PF < NB) {
+                        a[PF > 0 ? b % PF : 0] = rd(b + PF);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
                 }
             };
             half(std::integral_constant<int, 0>{});

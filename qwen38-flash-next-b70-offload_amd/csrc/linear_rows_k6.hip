@@ -1,0 +1,9 @@
+// The dense linear's product for more rows: (bitrate, codebook) (6, 1), (6, 0).
+#include "linear_rows.cuh"
+
+namespace exl3 {
+template void linear_rows_product<6, 1>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+                                         int64_t out_stride, hipStream_t s);
+template void linear_rows_product<6, 0>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+                                         int64_t out_stride, hipStream_t s);
+}  // namespace exl3

@@ -1014,6 +1014,54 @@ int exl3_linear_small(const void* x, int x_dtype, int64_t x_stride, int M, int k
     return e == hipSuccess ? EXL3_OK : hip_fail(e, "linear_small launch");
 }
 
+// the workspace of a linear_rows call: xh [S][M][k] fp16, then the partial sums [P][M][n] fp32 of its K-slices
+static size_t linear_rows_xh_bytes(int M, int k, int S) { return align256((size_t)S * M * k * 2); }
+size_t exl3_linear_rows_workspace(int M, int k, int n, int S, int width) {
+    if (M <= 0 || k <= 0 || n <= 0 || S <= 0 || (width != 128 && width != 256)) return 0;
+    const int P = linear_rows_slices(M, k, n, width);
+    return linear_rows_xh_bytes(M, k, S) + (P > 1 ? align256((size_t)P * M * n * 4) : 0);
+}
+
+int exl3_linear_rows(const void* x, int x_dtype, int64_t x_stride, int M, int k, int n, const void* trellis, int K,
+                     int cb, const void* suh, int S, const void* svh, const int64_t* group_bounds, int width, void* out,
+                     int out_dtype, int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream) {
+    if (int r = linear_dims("linear_rows", M, k, n, S)) return r;
+    if (!exl3_linear_supported(K, cb)) return fail(EXL3_EUNSUPPORTED, "linear_rows: K=%d cb=%d", K, cb);
+    if (x_dtype < EXL3_DT_F16 || x_dtype > EXL3_DT_F32 || out_dtype < EXL3_DT_F16 || out_dtype > EXL3_DT_F32)
+        return fail(EXL3_EINVAL, "linear_rows: dtype");
+    if ((width != 128 && width != 256) || n % width) return fail(EXL3_EINVAL, "linear_rows: width=%d n=%d", width, n);
+    if (M == 0) return EXL3_OK;
+    if (!x || !trellis || !suh || !svh || !group_bounds || !out) return fail(EXL3_EINVAL, "linear_rows: null pointer");
+    if (S > kLinMaxGroups) return fail(EXL3_EUNSUPPORTED, "linear_rows: S=%d > %d", S, kLinMaxGroups);
+    for (int g = 0; g <= S; ++g)
+        if (group_bounds[g] % width || (g ? group_bounds[g] < group_bounds[g - 1] : group_bounds[0] != 0) ||
+            (g == S && group_bounds[g] != n))
+            return fail(EXL3_EINVAL, "linear_rows: group_bounds [0, ..., n] in multiples of width");
+    if (x_stride < k || out_stride < n) return fail(EXL3_EINVAL, "linear_rows: row strides");
+    if ((int64_t)S * M * k * 2 >= (int64_t)1 << 31 || (int64_t)k * n / 8 * K >= (int64_t)1 << 31)
+        return fail(EXL3_EUNSUPPORTED, "linear_rows: S=%d M=%d k=%d n=%d exceeds 2 GiB of xh or trellis", S, M, k, n);
+    const size_t need = exl3_linear_rows_workspace(M, k, n, S, width);
+    if (!workspace || workspace_bytes < need)
+        return fail(EXL3_EWORKSPACE, "linear_rows: workspace %zu < %zu bytes", workspace_bytes, need);
+    LinearArgs a{};
+    a.x = x;
+    a.x_dt = x_dtype;
+    a.x_stride = x_stride;
+    a.M = M;
+    a.k = k;
+    a.n = n;
+    a.S = S;
+    a.tr = (const uint32_t*)trellis;
+    a.suh = (const _Float16*)suh;
+    a.svh = (const _Float16*)svh;
+    for (int g = 0; g < S; ++g) a.first[g] = (int)group_bounds[g];
+    a.xh = (_Float16*)workspace;
+    a.P = linear_rows_slices(M, k, n, width);
+    float* part = (float*)((uint8_t*)workspace + linear_rows_xh_bytes(M, k, S));
+    const hipError_t e = launch_linear_rows(K, cb, a, width, part, out, out_dtype, out_stride, (hipStream_t)stream);
+    return e == hipSuccess ? EXL3_OK : hip_fail(e, "linear_rows launch");
+}
+
 int exl3_had_in(const void* x, int x_dtype, int64_t x_stride, int M, int k, const void* suh, int S, void* xh,
                 void* stream) {
     if (int r = linear_dims("had_in", M, k, 128, S)) return r;

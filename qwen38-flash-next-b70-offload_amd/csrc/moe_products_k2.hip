@@ -1,0 +1,6 @@
+// The grouped experts' products at 2 bits.
+#include "moe_products.cuh"
+
+namespace exl3 {
+template void launch_products<2>(const GroupedArgs& a, bool y32, hipStream_t s);
+}  // namespace exl3

@@ -361,9 +361,11 @@ void linear_q8(const at::Tensor& x2, const at::Tensor& trellis, const at::Tensor
     }
 }
 
-// exl3_linear (exl3_ops.sycl:651-757): M <= small_m_max (at most 8 rows here) -> the fused path; otherwise the input
-// Hadamards, per shard group the reconstructed fp16 weights in slices of slice_n columns times xh[g] (a library
-// GEMM, fp16 output), then the output Hadamard
+// exl3_linear (exl3_ops.sycl:651-757): M <= small_m_max (at most 8 rows here) -> the fused path; otherwise, with shards of
+// whole 128-column blocks, exl3_linear_rows, which decodes the trellis inside the product (111 -> 26 us at 40 rows and
+// 689 -> 557 us at 8,192 rows of 2048 -> 12,288 against the following); else the input Hadamards, per shard group the
+// reconstructed fp16 weights in slices of slice_n columns times xh[g] (a library GEMM, fp16 output), then the output
+// Hadamard
 at::Tensor linear(at::Tensor x, at::Tensor trellis, at::Tensor suh, at::Tensor svh, at::Tensor shard_of_nb,
                   at::IntArrayRef group_bounds, int64_t K, int64_t cb, int64_t small_m_max, int64_t slice_n) {
     auto shape = x.sizes().vec();
@@ -384,6 +386,27 @@ at::Tensor linear(at::Tensor x, at::Tensor trellis, at::Tensor suh, at::Tensor s
                 "exl3xpu_C.linear: group_bounds [0, ..., n] with one group per suh row");
     if (g_int8.load() && cb == 2 && (K == 4 || K == 6) && M > 16) {     // exl3_ops.sycl:668
         linear_q8(x2, trellis, suh, svh, group_bounds, K, out);
+        return out.view(shape);
+    }
+    // (row slices keep xh below 2 GiB)
+    int64_t width = S <= 16 && k * n / 8 * K < (int64_t)1 << 31 && S * k <= (int64_t)1 << 22 ? 256 : 0;
+    for (int64_t g = 0; g < S && width; ++g) {
+        TORCH_CHECK(group_bounds[g] <= group_bounds[g + 1], "exl3xpu_C.linear: group_bounds not ascending");
+        width = group_bounds[g + 1] % 128 ? 0 : group_bounds[g + 1] % 256 ? 128 : width;
+    }
+    if (width) {
+        const int64_t step = std::min<int64_t>(M, std::max<int64_t>(128, (((int64_t)1 << 30) - 1) / (S * k) / 128 * 128));
+        const size_t wb = exl3_linear_rows_workspace((int)step, (int)k, (int)n, (int)S, (int)width);
+        auto ws = at::empty({(int64_t)wb}, x.options().dtype(at::kByte));
+        const int64_t esz = x2.element_size();
+        for (int64_t m0 = 0; m0 < M; m0 += step) {
+            const int64_t ms = std::min(step, M - m0);
+            check(exl3_linear_rows((const char*)x2.data_ptr() + m0 * k * esz, dtype_code(x2), k, (int)ms, (int)k, (int)n,
+                                   trellis.data_ptr(), (int)K, (int)cb, suh.data_ptr(), (int)S, svh.data_ptr(),
+                                   group_bounds.data(), (int)width, (char*)out.data_ptr() + m0 * n * esz,
+                                   dtype_code(out), n, ws.data_ptr(), wb, cur_stream(x2)),
+                  "exl3xpu_C.linear (rows)");
+        }
         return out.view(shape);
     }
     auto xh = at::empty({S, M, k}, x.options().dtype(at::kHalf));
