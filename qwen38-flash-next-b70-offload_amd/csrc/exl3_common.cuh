@@ -458,5 +458,11 @@ __device__ __forceinline__ void counter_reset(int* c) { __hip_atomic_store(c, 0,
 // global-address-space view of a generic pointer (global_load instead of flat_load)
 typedef const __attribute__((address_space(1))) uint32_t gu32_t;
 __device__ __forceinline__ gu32_t* as_global(const uint32_t* p) { return (gu32_t*)p; }
+// 8 fp16 values at any even address of global memory (a pointer read from a table would make it a flat load, which also
+// counts as an LDS access)
+typedef _Float16 half8_u __attribute__((ext_vector_type(8), aligned(2)));
+__device__ __forceinline__ half8_u ld_half8(const void* p) {
+    return *(const __attribute__((address_space(1))) half8_u*)(uintptr_t)p;
+}
 
 }  // namespace exl3

@@ -9,8 +9,6 @@
 
 namespace exl3 {
 
-typedef _Float16 half8_u __attribute__((ext_vector_type(8), aligned(2)));   // scales at any alignment
-
 // A workgroup of 2 CW waves: CW waves of 64 columns for each half of its K-slice (twice the waves per SIMD that the
 // columns alone give, at no traffic: the halves are summed in LDS). Each half is staged as a matrix of its own.
 template <int K, int CB, int NB, int CW>

@@ -21,12 +21,11 @@
 #include "exl3_geom.h"
 #include "exl3_kernels.h"
 #include "exl3_regb.cuh"
+#include "exl3_xh.cuh"
 
 #include <algorithm>
 
 namespace exl3 {
-
-typedef float float16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kPreThreads = 1024;
 
@@ -116,108 +115,66 @@ __device__ __forceinline__ void sort_wg(const GroupedArgs& A, int* off /* LDS [E
 }
 
 // ---- input Hadamards ---------------------------------------------------------------------------------------------------
-// xh[pick][pj][kb * 128 + n] = fp16(sum_k H[n][k] fp16(x[row][kb * 128 + k] suh_pj[kb * 128 + k]) / sqrt 128) as MFMA
-// products C^T = H128 xt^T (A fragments: two per-lane +-1 fragments and their negatives, from the bit split of
-// popc(n & k); B = 32 picks). One wave per (32 picks, projection, kbs 128-blocks), results through LDS in halves of 64
-// columns, so that 8 lanes store 128 contiguous bytes of a pick.
-constexpr int kXhRow = 64 + 8;                   // LDS row of one pick's half block (halfs, padded)
-typedef _Float16 half8_u __attribute__((ext_vector_type(8), aligned(2)));   // activations and blob vectors: any alignment
-typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
-
+// xh[pick][pj][kb * 128 ..] = fp16(H(fp16(x[row] suh_pj)) / sqrt 128), one wave per (4 picks, kbs 128-blocks) and both
+// projections: 16 lanes hold a pick's block, 8 values each (row_fwht128_signed). Few registers, no LDS, full cache lines
+// in and out. As MFMA products with H128 (32 picks per wave, through LDS twice, 128 VGPRs) the blocks of a wave ran one
+// after the other, 6 us each: 250-280 us at 8,192 tokens, 82 us at 2,048; so 201 and 57 us, with 671 MB written (107 us at
+// 6.3 TB/s) at 8,192.
 template <int DT>
-__device__ __forceinline__ void ld_x8(const void* x, size_t i, float (&v)[8]) {
-    if constexpr (DT == 2) {
-        const float4_u a = *(const float4_u*)((const float*)x + i), b = *(const float4_u*)((const float*)x + i + 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[j] = a[j];
-            v[4 + j] = b[j];
-        }
-    } else if constexpr (DT == 1) {
-        const u32x4_u w = *(const u32x4_u*)((const bf16_bits*)x + i);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[2 * j] = __uint_as_float(w[j] << 16);
-            v[2 * j + 1] = __uint_as_float(w[j] & 0xFFFF0000u);
-        }
-    } else {
-        const half8_u h = *(const half8_u*)((const half_t*)x + i);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (float)h[j];
-    }
-}
-
-template <int DT>
-__device__ __forceinline__ void xh_task(const GroupedArgs& A, int task, int kbs, half_t* tb) {
-    const int H = A.g.H, nkb = H / 128, nks = (nkb + kbs - 1) / kbs;
-    const int l = lane_id();
-    const int pj = task & 1, ks = (task >> 1) % nks, blk = (task >> 1) / nks;
-    half8_t hf[2][2];                            // [ks & 1][negated]: rows n' = l % 32, k' = 8 (l / 32) + j
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
+__device__ __forceinline__ void xh_task(const GroupedArgs& A, int task, int kbs) {
+    const int H = A.g.H, nkb = H / 128, nks = (nkb + kbs - 1) / kbs, l = lane_id();
+    const int ks = task % nks, p = task / nks * 4 + (l >> 4), c = (l & 15) * 8;
+    const int s = min(p, A.npairs - 1);          // (lanes past the end repeat the last pick and store nothing)
+    const size_t xo = (size_t)(s / A.topk) * A.x_stride + c;
+    const uint8_t* su = (const uint8_t*)A.ptrs[min(max(A.ids[s], 0), A.E - 1)] + A.g.off_suh_g + 2 * c;
+    half_t* o = A.xh + (size_t)s * 2 * H + c;
+    const float rs = row_sign() * kRsqrt128;
+    const int kb1 = min(nkb, (ks + 1) * kbs);
+    XRaw<DT> x;
+    half8_u sg, sv;
+    auto load = [&](int kb) {
+        ld_x8<DT>(A.x, xo + kb * 128, x);
+        sg = ld_half8(su + kb * 256);
+        sv = ld_half8(su + 2 * H + kb * 256);    // suh_u follows suh_g
+    };
+    load(ks * kbs);
+    for (int kb = ks * kbs; kb < kb1; ++kb) {
+        float g[8], u[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const bool neg = __popc((l & 31) & (b * 16 + (l >> 5) * 8 + j)) & 1;
-            hf[b][0][j] = neg ? (half_t)-1.0f : (half_t)1.0f;
-            hf[b][1][j] = neg ? (half_t)1.0f : (half_t)-1.0f;
+            g[j] = x_su<DT>(x, j, sg[j]);
+            u[j] = x_su<DT>(x, j, sv[j]);
         }
-    const int s0 = blk * 32, s = min(s0 + (l & 31), A.npairs - 1);     // (lanes past the end repeat the last pick)
-    const size_t xrow = (size_t)(s / A.topk) * A.x_stride;
-    const half_t* suh = (const half_t*)((const uint8_t*)A.ptrs[min(max(A.ids[s], 0), A.E - 1)] +
-                                        (pj ? A.g.off_suh_u : A.g.off_suh_g));
-    for (int kb = ks * kbs; kb < min(nkb, (ks + 1) * kbs); ++kb) {
-        half8_t bx[8];                           // xt fragments: k = 16 i + 8 (l / 32) .. + 7
+        load(min(kb + 1, nkb - 1));              // the next block's, while this one is transformed
+        row_fwht128_signed(g);
+        row_fwht128_signed(u);
+        half8_t og, ou;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int k = kb * 128 + i * 16 + (l >> 5) * 8;
-            float xv[8];
-            ld_x8<DT>(A.x, xrow + k, xv);
-            const half8_u sv = *(const half8_u*)(suh + k);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) bx[i][j] = to_half(xv[j] * (float)sv[j]);
+        for (int j = 0; j < 8; ++j) {
+            og[j] = to_half(g[j] * rs);
+            ou[j] = to_half(u[j] * rs);
         }
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {
-#pragma unroll
-            for (int n2 = 0; n2 < 2; ++n2) {
-                const int nb = 2 * hb + n2;
-                float16_t acc = float16_t{};
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(hf[i & 1][__popc(nb & (i >> 1)) & 1], bx[i], acc, 0, 0, 0);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {    // rows n = 32 nb + 8 q + 4 (l / 32) + 0..3
-                    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-                    *(half4_t*)(tb + (l & 31) * kXhRow + n2 * 32 + q * 8 + (l >> 5) * 4) =
-                        half4_t{to_half(acc[4 * q] * kRsqrt128), to_half(acc[4 * q + 1] * kRsqrt128),
-                                to_half(acc[4 * q + 2] * kRsqrt128), to_half(acc[4 * q + 3] * kRsqrt128)};
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {        // the wave's own LDS rows: 8 picks x 128 bytes per store
-                const int pr = r * 8 + (l >> 3), col = (l & 7) * 8;
-                const half8_t v = *(const half8_t*)(tb + pr * kXhRow + col);
-                if (s0 + pr < A.npairs)
-                    *(half8_t*)(A.xh + ((size_t)(s0 + pr) * 2 + pj) * H + kb * 128 + hb * 64 + col) = v;
-            }
+        if (p < A.npairs) {
+            *(half8_t*)(o + kb * 128) = og;
+            *(half8_t*)(o + H + kb * 128) = ou;
         }
     }
 }
 
-__global__ void __launch_bounds__(kPreThreads) grouped_pre_kernel(GroupedArgs A, int ntask, int kbs) {
-    __shared__ __align__(16) half_t tbuf[kPreThreads / 64][32 * kXhRow];
+__global__ void __launch_bounds__(kPreThreads) __attribute__((amdgpu_waves_per_eu(8)))
+grouped_pre_kernel(GroupedArgs A, int ntask, int kbs) {
+    __shared__ int off[kMaxExperts];
     __shared__ uint64_t sw[17];
     if (blockIdx.x == 0) {
-        sort_wg(A, (int*)tbuf, sw);
+        sort_wg(A, off, sw);
         return;
     }
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int task = (blockIdx.x - 1) * (kPreThreads / 64) + wv;
-    if (task >= ntask) return;
-    if (A.x_dt == 1) xh_task<1>(A, task, kbs, tbuf[wv]);
-    else if (A.x_dt == 2) xh_task<2>(A, task, kbs, tbuf[wv]);
-    else xh_task<0>(A, task, kbs, tbuf[wv]);
+    if (task >= ntask) return;                   // (whole waves: the transforms need every lane)
+    if (A.x_dt == 1) xh_task<1>(A, task, kbs);
+    else if (A.x_dt == 2) xh_task<2>(A, task, kbs);
+    else xh_task<0>(A, task, kbs);
 }
 
 // out[m][h] = sum over the row's picks, in pick order, of y[m topk + k][h]; one thread per 8 columns. The picks' rows are
@@ -300,10 +257,12 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
     a.xh = (half_t*)take(np * 4 * a.g.H);
     a.abuf = (half_t*)take(np * 2 * a.g.I);
     a.y = take(np * a.g.H * (y32 ? 4 : 2));
-    const int nkb = a.g.H / 128, nblk = (a.npairs + 31) / 32;
-    int kbs = 1;                                 // 128-blocks per wave
-    while (kbs < nkb && 2 * nblk * ((nkb + kbs - 1) / kbs) > 65536) kbs *= 2;
-    const int ntask = 2 * nblk * ((nkb + kbs - 1) / kbs);
+    const int nkb = a.g.H / 128, nq = (a.npairs + 3) / 4;
+    // 128-blocks per wave: one while the waves do not fill the chip several times over, then up to 4, which hides a
+    // wave's own table lookups (8,192 tokens: 1 / 2 / 4 / 8 blocks 230 / 207 / 201 / 207 us; 16 rows: 5.4 / 5.6 / 8.6 us)
+    int kbs = 1;
+    while (kbs < 4 && nq * ((nkb + kbs - 1) / kbs) > 32768) kbs *= 2;
+    const int ntask = nq * ((nkb + kbs - 1) / kbs);
     hipLaunchKernelGGL(grouped_pre_kernel, dim3(1 + (unsigned)((ntask + 15) / 16)), dim3(kPreThreads), 0, s, a, ntask, kbs);
     switch (a.g.K) {
         case 2: launch_products<2>(a, y32, s); break;

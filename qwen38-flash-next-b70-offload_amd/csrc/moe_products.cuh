@@ -10,8 +10,6 @@
 
 namespace exl3 {
 
-typedef _Float16 half8_u __attribute__((ext_vector_type(8), aligned(2)));   // blob vectors: any alignment
-
 template <int NB> constexpr int kMoePf = NB >= 5 && NB <= 8 ? 4 : 0;
 constexpr int kMoeSd = 1;                        // chunks of A in flight in registers (the accumulators leave no room)
 constexpr int kEpRow = 260;                      // floats per row of the [16][256] epilogue tile (16-byte reads of 4 rows
@@ -94,9 +92,9 @@ __device__ __forceinline__ void gateup_item(const GroupedArgs& A, int e, int s0,
         __syncthreads();
         if (wv < 4) {                            // 4 rows per wave, 16 lanes x 8 columns per row
             const int rr = wv * 4 + (l >> 4), row = 16 * b + rr;
-            const half8_u hg = *(const half8_u*)((const half_t*)(base + A.g.off_svh_g) + cb8);
-            const half8_u hu = *(const half8_u*)((const half_t*)(base + A.g.off_svh_u) + cb8);
-            const half8_u hd = *(const half8_u*)((const half_t*)(base + A.g.off_suh_d) + cb8);
+            const half8_u hg = ld_half8(base + A.g.off_svh_g + 2 * cb8);
+            const half8_u hu = ld_half8(base + A.g.off_svh_u + 2 * cb8);
+            const half8_u hd = ld_half8(base + A.g.off_suh_d + 2 * cb8);
             float g[8], u[8], av[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) g[j] = u[j] = 0.f;
@@ -157,9 +155,9 @@ __device__ __forceinline__ void gateup_rows(const GroupedArgs& A, int e, int s0,
                                           soff, H / 64, pj, lds, acc);
     // 16 rows per round through one of two tiles [16][gate 32 WV | up 32 WV]: 16 lanes per (row, 128 columns)
     const int un = threadIdx.x >> 4, rr = un & 15, cb = (un >> 4) * 128 + (l & 15) * 8, ci = nb * 32 * WV + cb;
-    const half8_u hg = *(const half8_u*)((const half_t*)(base + A.g.off_svh_g) + ci);
-    const half8_u hu = *(const half8_u*)((const half_t*)(base + A.g.off_svh_u) + ci);
-    const half8_u hd = *(const half8_u*)((const half_t*)(base + A.g.off_suh_d) + ci);
+    const half8_u hg = ld_half8(base + A.g.off_svh_g + 2 * ci);
+    const half8_u hu = ld_half8(base + A.g.off_svh_u + 2 * ci);
+    const half8_u hd = ld_half8(base + A.g.off_suh_d + 2 * ci);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         float* ep = (float*)lds + (b & 1) * 16 * kEpRowW<WV>;
@@ -233,7 +231,7 @@ __device__ __forceinline__ void down_rows(const GroupedArgs& A, int e, int s0, i
         for (int i = 0; i < 2; ++i) {
             const int un = (threadIdx.x >> 4) + i * 4 * WV, rr = un & 15, cb = (un >> 4) * 128 + (l & 15) * 8;
             const int row = 16 * b + rr, ch = nt * 64 * WV + cb;
-            const half8_u hs = *(const half8_u*)((const half_t*)(base + A.g.off_svh_d) + ch);
+            const half8_u hs = ld_half8(base + A.g.off_svh_d + 2 * ch);
             const int pk = A.perm[s0 + min(row, rows - 1)];
             const float pw = A.w[pk];
             float v[8];
