@@ -111,9 +111,10 @@ size_t exl3_moe_forward_workspace(int M, int H, int I, int topk, int n_experts);
 /* moe_forward (a8:1221-1225 -> moe_forward_impl a8:1263-1314): out[m] = sum_k w[m,k] * expert(ids[m,k])(x[m]).
  * x, out: [M, H] with row strides, dtype EXL3_DT_*; ids int32 / w fp32 [M, topk] contiguous; ptrs int64 [n_experts]
  * blob addresses (device slots or device-mapped pinned host memory). Small decode calls run the fused decode kernel;
- * with H % 256 == 0, decode calls from topk * M * I = 60,000 on and every call of M >= prefill_min_m (or of more than
- * 1024 picks or 256 rows, which need it) run the grouped kernels (moe_prefill a8:792-828): token sort, the experts'
- * trellis decoded into MFMA registers once for all their rows, combine; y in fp16 from prefill_min_m on. */
+ * with H % 256 == 0, decode calls from topk * M * I = 56,000 on (49,000 for I >= 1024) and every call of
+ * M >= prefill_min_m (or of more than 1024 picks or 256 rows, which need it) run the grouped kernels (moe_prefill
+ * a8:792-828): token sort, the experts' trellis decoded into MFMA registers once for all their rows, combine; y in
+ * fp16 from prefill_min_m on. */
 int exl3_moe_forward(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
                      const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
                      int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream);

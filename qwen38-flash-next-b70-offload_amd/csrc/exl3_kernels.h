@@ -112,7 +112,6 @@ constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // the dense EXL3 linear (linear.hip): out[M, n] = svh * H(sum_k xh[shard of n][m][k] W[k][n]) / sqrt 128
 constexpr int kLinMaxRows = 8;       // rows of the fused small-M path
-constexpr int kLinMaxGroups = 16;    // shards of a linear_rows call
 struct LinearArgs {
     const void* x; int x_dt; int64_t x_stride;     // activations [M, k]
     int M, k, n, S;                                // rows, input and output features, shards
@@ -120,7 +119,6 @@ struct LinearArgs {
     const _Float16* suh;                           // [S][k]
     const _Float16* svh;                           // [n]
     const int32_t* shard_of_nb;                    // [n/128]
-    int first[kLinMaxGroups];                      // linear_rows: every shard's first column
     _Float16* xh;                                  // [S][M][k] (the large-M path's input Hadamards)
     uint64_t* part;                                // [P][M][n] tagged partial sums over the K-slices: zero on
                                                    // entry, left zero
@@ -133,15 +131,19 @@ hipError_t launch_linear_had_in(const LinearArgs& a, hipStream_t s);
 // codebook cb: 2 mul1 (K = 2..6), 1 mcg or 0 3inst (K = 4, 6)
 hipError_t launch_linear_small(int K, int cb, const LinearArgs& a, void* out, int out_dt, int64_t out_stride,
                                hipStream_t s);
+constexpr int kLinMaxGroups = 16;    // shards of a linear_rows call
+struct LinearRowsArgs : LinearArgs {
+    int first[kLinMaxGroups];                      // every shard's first column
+};
 // the linear for more rows (linear_rows.hip): xh [S][M][k] and part fp32 [P][M][n] (P > 1) are workspaces; every shard's
 // columns are a multiple of width (256 or 128); S M k and k n K / 8 bytes below 2 GiB
 // 16-row blocks of a workgroup: up to 64 rows in one tile, above that tiles of 128 (each tile decodes the weights again)
 static inline int linear_rows_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
 int linear_rows_slices(int M, int k, int n, int width);
 template <int K, int CB>
-void linear_rows_product(const LinearArgs& a, int width, float* part, void* out, int out_dt, int64_t out_stride,
+void linear_rows_product(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt, int64_t out_stride,
                          hipStream_t s);
-hipError_t launch_linear_rows(int K, int cb, const LinearArgs& a, int width, float* part, void* out, int out_dt,
+hipError_t launch_linear_rows(int K, int cb, const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                               int64_t out_stride, hipStream_t s);
 // out = svh * H(sum of P parts) / sqrt 128; parts fp32 (y_half 0) or one fp16 matrix (y_half 1, P 1)
 hipError_t launch_linear_had_out(const void* parts, int y_half, int P, int M, int n, const _Float16* svh, void* out,

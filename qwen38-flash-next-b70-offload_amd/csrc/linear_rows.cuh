@@ -13,7 +13,7 @@ namespace exl3 {
 // columns alone give, at no traffic: the halves are summed in LDS). Each half is staged as a matrix of its own.
 template <int K, int CB, int NB, int CW>
 __global__ void __launch_bounds__(128 * CW) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 4 : NB <= 4 ? 3 : 2)))
-lin_rows_kernel(LinearArgs A, float* part, void* out, int out_dt, int64_t out_stride, int vec) {
+lin_rows_kernel(LinearRowsArgs A, float* part, void* out, int out_dt, int64_t out_stride, int vec) {
     constexpr int WV = 2 * CW;
     using B = RegB<K, true, CB>;
     using U = AUnits<NB, WV, 2>;
@@ -92,7 +92,7 @@ lin_rows_kernel(LinearArgs A, float* part, void* out, int out_dt, int64_t out_st
 }
 
 template <int K, int CB>
-void linear_rows_product(const LinearArgs& a, int width, float* part, void* out, int out_dt, int64_t out_stride,
+void linear_rows_product(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt, int64_t out_stride,
                         hipStream_t s) {
     const int nb = linear_rows_blocks(a.M), vec = (out_stride & 7) == 0 && ((uintptr_t)out & 15) == 0;
     const dim3 grid((unsigned)((a.n / width) * a.P * ((a.M + 16 * nb - 1) / (16 * nb))));

@@ -64,10 +64,11 @@ int linear_rows_slices(int M, int k, int n, int width) {
     return nkb <= 4 ? 1 : std::max(1, std::min(std::min(8, nkb / 2), 256 / wgs));
 }
 
-hipError_t launch_linear_rows(int K, int cb, const LinearArgs& a, int width, float* part, void* out, int out_dt,
+hipError_t launch_linear_rows(int K, int cb, const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                               int64_t out_stride, hipStream_t s) {
     const int tasks = (a.M + 3) / 4 * (a.k / 128);
-    hipLaunchKernelGGL(lin_xh_kernel, dim3((unsigned)((tasks + kLxWaves - 1) / kLxWaves)), dim3(64 * kLxWaves), 0, s, a);
+    hipLaunchKernelGGL(lin_xh_kernel, dim3((unsigned)((tasks + kLxWaves - 1) / kLxWaves)), dim3(64 * kLxWaves), 0, s,
+                       (const LinearArgs&)a);
     switch (cb * 8 + K) {
         case 16 + 2: linear_rows_product<2, 2>(a, width, part, out, out_dt, out_stride, s); break;
         case 16 + 3: linear_rows_product<3, 2>(a, width, part, out, out_dt, out_stride, s); break;

@@ -2,10 +2,10 @@
 #include "linear_rows.cuh"
 
 namespace exl3 {
-template void linear_rows_product<4, 2>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+template void linear_rows_product<4, 2>(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                                          int64_t out_stride, hipStream_t s);
-template void linear_rows_product<4, 1>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+template void linear_rows_product<4, 1>(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                                          int64_t out_stride, hipStream_t s);
-template void linear_rows_product<4, 0>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+template void linear_rows_product<4, 0>(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                                          int64_t out_stride, hipStream_t s);
 }  // namespace exl3

@@ -2,8 +2,8 @@
 #include "linear_rows.cuh"
 
 namespace exl3 {
-template void linear_rows_product<5, 2>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+template void linear_rows_product<5, 2>(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                                          int64_t out_stride, hipStream_t s);
-template void linear_rows_product<6, 2>(const LinearArgs& a, int width, float* part, void* out, int out_dt,
+template void linear_rows_product<6, 2>(const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,
                                          int64_t out_stride, hipStream_t s);
 }  // namespace exl3

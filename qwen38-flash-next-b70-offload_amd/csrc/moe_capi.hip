@@ -259,13 +259,13 @@ static bool exceeds_decode(int M, int topk) { return (int64_t)M * topk > kMaxPai
 static bool use_prefill(int M, int topk) { return M >= g_cfg.prefill_min_m || exceeds_decode(M, topk); }
 
 // the grouped kernels (moe_grouped.hip) decode each expert's weights once for all of its picks, the fused decode kernel
-// once per pick: they take every call of the prefill sizes, and the decode sizes from picks * I = 60,000 on. Below it
-// the fused kernel's single launch is faster: at H 2048 / I 512, top-10, 54 us against 73 us for 8 rows of distinct
-// experts (80 picks) and 104 against 74 us for 16 Zipf rows; at H 4096 / I 1536, top-8, 66 against 85 us for 2 rows and
-// 184 against 151 us for 6.
-constexpr int64_t kGroupedMinWork = 60000;
+// once per pick: they take every call of the prefill sizes, and the decode sizes from picks * I = 56,000 on (49,000 for
+// experts of I >= 1024). Below that the fused kernel's single launch is faster, or the experts' workgroups divide badly
+// over the CUs: at H 2048 / I 512, top-10, 54 us against 67 us for 8 rows of distinct experts (80 picks), but 79 against
+// 56 us for 12 Zipf rows; at H 4096 / I 1536, top-8, K 4, 97 against 109 us for 3 rows and 126 against 110 us for 4.
 static bool use_grouped(int M, int topk, int H, int I) {
-    return H % 256 == 0 && (use_prefill(M, topk) || (int64_t)M * topk * I >= kGroupedMinWork);
+    const int64_t min_work = I >= 1024 ? 49000 : 56000;
+    return H % 256 == 0 && (use_prefill(M, topk) || (int64_t)M * topk * I >= min_work);
 }
 // the picks' outputs stay fp32 at the decode sizes, and are fp16 at the prefill sizes (as the reference keeps them)
 static bool grouped_y32(int M, int topk) { return !use_prefill(M, topk); }
@@ -1043,7 +1043,7 @@ int exl3_linear_rows(const void* x, int x_dtype, int64_t x_stride, int M, int k,
     const size_t need = exl3_linear_rows_workspace(M, k, n, S, width);
     if (!workspace || workspace_bytes < need)
         return fail(EXL3_EWORKSPACE, "linear_rows: workspace %zu < %zu bytes", workspace_bytes, need);
-    LinearArgs a{};
+    LinearRowsArgs a{};
     a.x = x;
     a.x_dt = x_dtype;
     a.x_stride = x_stride;

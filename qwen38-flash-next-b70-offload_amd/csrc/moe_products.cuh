@@ -243,6 +243,44 @@ __device__ __forceinline__ void down_rows(const GroupedArgs& A, int e, int s0, i
     }
 }
 
+// an item of one block: 4 waves of 64 columns (256 of H) in each of KS K-slices
+template <int K, int KS, typename TY>
+__device__ __forceinline__ void down_item(const GroupedArgs& A, int e, int s0, int rows, int nt, float* ep) {
+    const int I = A.g.I, H = A.g.H, tiles_n = H / 16, l = lane_id();
+    const int wv = uni(threadIdx.x >> 6), wc = wv & 3, ks = wv >> 2;
+    using B = RegB<K, false, 2>;
+    const uint8_t* base = expert_base(A, e);
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base) + A.g.gu_bytes, (short)0,
+                                                      (int)A.g.d_bytes, 0x00020000);
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(A.abuf, (short)0, A.npairs * 2 * I, 0x00020000);
+    const int m = l & 15;
+    const uint32_t aoff[1] = {m < rows ? (uint32_t)A.perm[s0 + m] * 2u * I + B::a_lane_off() : kOob};
+    float4_t acc[1][2][2];
+    acc[0][0][0] = acc[0][0][1] = acc[0][1][0] = acc[0][1][1] = float4_t{};
+    const int nch = I / 64;
+    regb_core<K, 1, false, 2>(rw, B::lane_off(tiles_n, nt * 16 + wc * 4), tiles_n, ra, aoff, nch * ks / KS,
+                              nch * (ks + 1) / KS, acc);
+    stash<K>(acc[0], ep + ks * 16 * kEpRow, wc);
+    __syncthreads();
+    // 16 rows x 2 halves of 128 columns, 16 lanes each
+#pragma unroll
+    for (int u0 = 0; u0 < 32; u0 += 16 * KS) {
+        const int un = u0 + (threadIdx.x >> 4), rr = un & 15, cb = (un >> 4) * 128 + (l & 15) * 8, ch = nt * 256 + cb;
+        const int pk = A.perm[s0 + min(rr, rows - 1)];
+        const half8_u hs = ld_half8(base + A.g.off_svh_d + 2 * ch);
+        const float pw = A.w[pk];
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; ++k)             // the K-slices in order
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] += ep[(k * 16 + rr) * kEpRow + cb + j];
+        row_fwht128_signed(v);
+        if (rr < rows) st_y<TY>(A.y, (size_t)pk * H + ch, v, row_sign() * kRsqrt128 * pw, hs);
+    }
+}
+
 // One launch per product (two launches, one per item size, left the chip idle behind the longest item of each: a batch
 // of 64 rows took 193 us in two, 132 us in one). !BIG (items of up to 4 blocks): 4 waves per SIMD; the items of several blocks come first, then
 // those of one. BIG (items of up to 12 blocks): 2 waves per SIMD, block counts below 9 rounded up to 4, 6 or 8.
@@ -287,13 +325,29 @@ __global__ void __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(BI
 grouped_down_kernel(GroupedArgs A) {
     constexpr int kLds = std::max(2 * AUnits<BIG ? 12 : 4, WV, 1>::kBuf, 2 * 16 * kEpRowW<WV> * 4);
     __shared__ __align__(16) uint8_t lds[kLds];
+    // the items of one block apart, at the decode sizes (fp32 outputs): there are few, and 256 columns x 2 K-slices spread
+    // them better than 512 columns (16 rows 23 -> 19 us, 6 rows of wide experts 62 -> 45 us); 512 experts of 5 rows fill
+    // the chip either way and take 97 us in 512 columns against 99
+    constexpr bool kOne = !BIG && sizeof(TY) == 4;
+    const int nblk = A.g.H / (64 * WV), nmany = uni(A.n_items[kOne ? 1 : 0]);
+    const int blk = blockIdx.x, bmany = (nmany + 7) / 8 * 8 * nblk;
     int a, nt;
-    gr_block(blockIdx.x, A.g.H / (64 * WV), a, nt);
-    if (a >= A.n_items[0]) return;
+    if (!kOne || blk < bmany) {
+        gr_block(blk, nblk, a, nt);
+        if (a >= nmany) return;
+    } else {
+        if constexpr (kOne) {
+            gr_block(blk - bmany, A.g.H / 256, a, nt);
+            a += nmany;
+            if (a >= uni(A.n_items[0])) return;
+            down_item<K, WV / 4, TY>(A, uni(A.it_expert[a]), uni(A.it_start[a]), uni(A.it_cnt[a]), nt, (float*)lds);
+        }
+        return;
+    }
     const int e = uni(A.it_expert[a]), s0 = uni(A.it_start[a]), rows = uni(A.it_cnt[a]), bl = (rows + 15) >> 4;
     if constexpr (!BIG) {
-        if (bl == 1) down_rows<K, 1, WV, false, TY>(A, e, s0, rows, nt, lds);
-        else if (bl == 2) down_rows<K, 2, WV, true, TY>(A, e, s0, rows, nt, lds);
+        if (!kOne && bl == 1) down_rows<K, 1, WV, false, TY>(A, e, s0, rows, nt, lds);
+        else if (bl <= 2) down_rows<K, 2, WV, true, TY>(A, e, s0, rows, nt, lds);
         else if (bl == 3) down_rows<K, 3, WV, true, TY>(A, e, s0, rows, nt, lds);
         else down_rows<K, 4, WV, true, TY>(A, e, s0, rows, nt, lds);
     } else {
@@ -324,8 +378,9 @@ void launch_products(const GroupedArgs& a, bool y32, hipStream_t s) {
     }
     auto down = [&](auto ty) {
         using TY = decltype(ty);
-        if (H % 512 == 0) run(grouped_down_kernel<K, 8, false, TY>, g8(mi) * (H / 512), 512);
-        else run(grouped_down_kernel<K, 4, false, TY>, g8(mi) * (H / 256), 256);
+        const unsigned one = g8(std::min<size_t>(np, a.E)) * (H / 256);
+        if (H % 512 == 0) run(grouped_down_kernel<K, 8, false, TY>, y32 ? many * (H / 512) + one : g8(mi) * (H / 512), 512);
+        else run(grouped_down_kernel<K, 4, false, TY>, y32 ? many * (H / 256) + one : g8(mi) * (H / 256), 256);
     };
     if (big) run(grouped_down_kernel<K, 8, true, half_t>, g8(mi) * (H / 512), 512);
     else if (y32) down(float{});
