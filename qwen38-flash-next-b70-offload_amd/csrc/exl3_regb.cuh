@@ -258,7 +258,8 @@ __device__ __forceinline__ void regb_lds_core(R rw, uint32_t woff, int tiles_n, 
                 }
                 const uint8_t* af = a0 + a_slot16(l & 15, B::F8 ? 2 * q + f : 4 * f + q);
                 auto rd = [&](int b) { return *(const half8_t*)(af + b * 16 * 128); };
-                half8_t w[2][2], a[PF > 0 ? PF : 1];
+                constexpr int kPf = PF > 0 ? PF : 1;
+                half8_t w[2][2], a[kPf];
                 if constexpr (PF > 0) {          // before the decode, so that it covers their latency
 #pragma unroll
                     for (int b = 0; b < PF; ++b) a[b] = rd(b);
@@ -271,14 +272,14 @@ __device__ __forceinline__ void regb_lds_core(R rw, uint32_t woff, int tiles_n, 
                 }
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const half8_t ab16 = PF > 0 ? a[PF > 0 ? b % PF : 0] : rd(b);
+                    const half8_t ab16 = PF > 0 ? a[b % kPf] : rd(b);
 #pragma unroll
                     for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
                             acc[b][cc][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ab16, w[cc][h], acc[b][cc][h], 0, 0, 0);
                     if (PF > 0 && b + PF < NB) {
-                        a[PF > 0 ? b % PF : 0] = rd(b + PF);
+                        a[b % kPf] = rd(b + PF);
                         __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
                         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                     }
