@@ -101,6 +101,7 @@ struct GroupedArgs {
     int rmax;                                      // rows of an item at most (64 or 192)
     int* it_expert; int* it_start; int* it_cnt;    // items: up to rmax sorted positions of one expert, longest first
     int* n_items;                                  // [2] items, and those of more than 16 rows (the first ones)
+    _Float16* suh;                                 // [E][2][H] input scales of the experts in use, or null: in the blobs
     _Float16* xh;                                  // [npairs][2][H] input Hadamards (gate, up)
     _Float16* abuf;                                // [npairs][I]
     void* y;                                       // [npairs][H] fp32 or fp16, routing weight applied

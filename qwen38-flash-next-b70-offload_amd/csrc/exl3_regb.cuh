@@ -6,7 +6,8 @@
 // that the A fragments share. A period holds two columns (c and c + 8 of a tile: h = 0, 1), so lane n decodes tile-
 // column n >> 3 of a pair and column n & 7 (+ 8 h), and the k-groups q are chosen so that a lane's 8 rows of a column
 // come from its own words:
-//   V = 32 (K = 3, 5): one period = all 16 rows. q = tile-row of the chunk, fragment f = rows 8 f .. 8 f + 7 of it.
+//   V = 32 (K = 3, 5): one period = all 16 rows. q = tile-row of the chunk (in the order of krow), fragment f = rows
+//     8 f .. 8 f + 7 of it.
 //   V = 16 (K = 2, 6) and V = 8 (K = 4): f = pair of tile-rows, q >> 1 the tile-row of the pair and b = q & 1 the rows
 //     {4 b .. 4 b + 3, 8 + 4 b .. 8 + 4 b + 3}: one period at V = 16, two neighbouring ones at V = 8.
 #pragma once
@@ -33,14 +34,19 @@ struct RegB {
     static constexpr int D = GM::D, V = GM::V, G = GM::G, W = GM::W;
     static constexpr bool F8 = V == 32;
     static constexpr int NP = V == 8 ? 2 : 1;        // periods of a lane per tile
+    // PLANAR4 words of K = 3: a load takes whole 128-byte lines, 2 tile-rows x 4 tile-columns, and one permlane16 swap per
+    // word of the two loads gives the lanes their tile-column pairs, with the tile-rows in the order 0, 2, 1, 3. Loads
+    // of 2 columns of 4 tile-rows take half lines: with a third of the experts in host memory 50.6 GB/s over PCIe
+    // against 52.9 with whole lines, 301 tokens 254 against 250 us
+    static constexpr bool SWAP = F8 && !NAT;
     static constexpr int SPC = F8 ? 1 : 2;           // steps (tile-row groups) of a chunk
     static constexpr int NW = SPC * 2 * NP * D;      // words of a lane per chunk
     static_assert(V == 32 || V == 16 || V == 8, "periods of 32, 16 or 8 values");
 
     // byte offset of this lane's first word of chunk 0 in the strip of tile-columns ct0 .. ct0 + 3
     __device__ __forceinline__ static uint32_t lane_off(int tiles_n, int ct0) {
-        const int l = lane_id(), q = l >> 4, c = (l >> 3) & 1, n = l & 7;
-        const int r = F8 ? q : q >> 1;
+        const int l = lane_id(), q = l >> 4, c = (l >> 3) & (SWAP ? 3 : 1), n = l & 7;
+        const int r = SWAP ? l >> 5 : F8 ? q : q >> 1;
         const int p = F8 ? n : (V == 16 ? 2 * n + (q & 1) : 4 * n + 2 * (q & 1));
         return 4u * (uint32_t)(NAT ? word_off_nat<K>(r, tiles_n, ct0 + c, p, 0) : word_off<K>(r, tiles_n, ct0 + c, p, 0));
     }
@@ -48,24 +54,51 @@ struct RegB {
     __device__ __forceinline__ static uint32_t chunk_bytes(int tiles_n) { return 16u * (uint32_t)tiles_n * W; }
 
     // the words of the chunk at byte offset off (lane_off + chunk * chunk_bytes; an offset past the descriptor's range
-    // reads zero without touching memory): order [step][column pair][period][word]
+    // reads zero without touching memory)
     template <typename R>
     __device__ __forceinline__ static void load(uint32_t (&w)[NW], R rsrc, uint32_t off, int tiles_n) {
         constexpr int kTwoTiles = NAT || D == 1 ? 2 * W : 2 * G;           // words from column pair 0 to 1
         constexpr int kPlane = NAT || D == 1 ? 1 : 4 * G;                  // words from word i to i + 1 of a period
+        if constexpr (SWAP) {                        // order [tile-row pair][word], see arrange
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < D; ++i)
+                    w[h * D + i] = __builtin_amdgcn_raw_buffer_load_b32(
+                        rsrc, (int)(off + h * 8u * (uint32_t)tiles_n * W + 4u * (i * kPlane)), 0, 2);   // 2: nt
+            return;
+        }
 #pragma unroll
         for (int s = 0; s < SPC; ++s) {
             const uint32_t o = off + (s ? 8u * (uint32_t)tiles_n * W : 0u);
 #pragma unroll
-            for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-                for (int j = 0; j < NP; ++j)
+            for (int cc = 0; cc < 2; ++cc) {
+                uint32_t* v = w + (s * 2 + cc) * NP * D;
+                if constexpr (NP == 2) {             // the two neighbouring words in one load
+                    const auto t = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)(o + 4u * cc * kTwoTiles), 0, 2);
+                    v[0] = t[0];
+                    v[1] = t[1];
+                } else {
 #pragma unroll
                     for (int i = 0; i < D; ++i)
-                        w[((s * 2 + cc) * NP + j) * D + i] = __builtin_amdgcn_raw_buffer_load_b32(
-                            rsrc, (int)(o + 4u * (cc * kTwoTiles + j * D + i * kPlane)), 0, 2);   // 2: nt
+                        v[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(o + 4u * (cc * kTwoTiles + i * kPlane)), 0, 2);
+                }
+            }
         }
     }
+    // the loaded words into the order [step][column pair][period][word] (before prep, once they are needed)
+    __device__ __forceinline__ static void arrange(uint32_t (&w)[NW]) {
+        if constexpr (SWAP) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) {
+                const auto t = __builtin_amdgcn_permlane16_swap(w[i], w[D + i], false, false);
+                w[i] = t[0];
+                w[D + i] = t[1];
+            }
+        }
+    }
+    // tile-row of k-group q (V = 32)
+    __device__ __forceinline__ static int krow(int q) { return SWAP ? ((q & 1) << 1) | (q >> 1) : q; }
 
     // the lane holding the period before this lane's first one (the trellis is circular in a tile)
     __device__ __forceinline__ static int prev_lane() {
@@ -105,7 +138,7 @@ struct RegB {
     // byte offset of this lane's A elements within a row (fp16, chunk 0, fragment 0)
     __device__ __forceinline__ static uint32_t a_lane_off() {
         const int q = lane_id() >> 4;
-        return F8 ? 32u * q : 32u * (q >> 1) + 8u * (q & 1);
+        return F8 ? 32u * krow(q) : 32u * (q >> 1) + 8u * (q & 1);
     }
     // A fragment f at row byte offset off (row start + a_lane_off) of the chunk at byte k0
     template <int f, typename R>
@@ -152,6 +185,7 @@ __device__ __forceinline__ void regb_core(R rw, uint32_t woff, int tiles_n, R ra
             if (c + j >= c1) break;
             const int kn = min(c + j + 1, c1 - 1) * 128;               // the next chunk's A (the last one's again)
             typename B::Dec d[2];
+            B::arrange(wd[j]);
             auto half = [&](auto F) {
                 constexpr int f = decltype(F)::value;
                 if (B::F8 ? f == 0 : true) {
@@ -250,13 +284,14 @@ __device__ __forceinline__ void regb_lds_core(R rw, uint32_t woff, int tiles_n, 
             stage_load((j + 1) % SD, c + j + 1 + SD);
             const uint8_t* a0 = ab + (j & 1) * U::kBuf;
             typename B::Dec d[2];
+            B::arrange(wd[j]);
             auto half = [&](auto F) {
                 constexpr int f = decltype(F)::value;
                 if (B::F8 ? f == 0 : true) {
                     B::prep(d[0], wd[j], B::F8 ? 0 : f, 0, src);
                     B::prep(d[1], wd[j], B::F8 ? 0 : f, 1, src);
                 }
-                const uint8_t* af = a0 + a_slot16(l & 15, B::F8 ? 2 * q + f : 4 * f + q);
+                const uint8_t* af = a0 + a_slot16(l & 15, B::F8 ? 2 * B::krow(q) + f : 4 * f + q);
                 auto rd = [&](int b) { return *(const half8_t*)(af + b * 16 * 128); };
                 constexpr int kPf = PF > 0 ? PF : 1;
                 half8_t w[2][2], a[kPf];

@@ -1,6 +1,7 @@
 // Routed experts with the picks grouped by expert (decode batches and prompts): every expert's trellis is decoded once
 // per item of up to 64 or 192 rows, straight into MFMA B registers (exl3_regb.cuh).
 //
+//   scales   above 16 picks per expert: the input scales of the experts in use, once each, into the workspace
 //   pre      one launch: workgroup 0 sorts the picks by expert and cuts them into items (longest first), the others
 //            write the input Hadamards xh of every (pick, projection), which need no sort
 //   gate/up  per (item, 32 WV columns of I), WV waves of 64 columns, half of them on each projection; the rows gathered
@@ -114,6 +115,35 @@ __device__ __forceinline__ void sort_wg(const GroupedArgs& A, int* off /* LDS [E
     each([&](int i, int e) { A.perm[atomicAdd(&off[e], 1)] = i; });
 }
 
+// ---- input scales ------------------------------------------------------------------------------------------------------
+// The input Hadamards run in pick order and read an expert's input scales for each of its picks: 8 KB per pick and expert
+// of H 2048. That is cache traffic for an expert in HBM, but host memory is not cached, so with a third of 512 experts
+// read over PCIe and 160 picks per expert it was 230 MB next to the 412 MB of their records (8,192 tokens 12.7 ms per
+// layer, 8.2 ms with the copies and with down's output scales loaded once; with every expert in HBM 1.09 ms either way). So each expert's scales are copied once: a workgroup per kScaleExperts experts looks for
+// them in the ids (an expert without picks may have no blob) and copies those that it finds.
+constexpr int kScaleExperts = 4;
+__global__ void __launch_bounds__(1024) grouped_scales_kernel(GroupedArgs A) {
+    __shared__ int used[kScaleExperts];
+    const int e0 = blockIdx.x * kScaleExperts, t = threadIdx.x;
+    if (t < kScaleExperts) used[t] = 0;
+    __syncthreads();
+    for (int i0 = t; i0 < A.npairs; i0 += 8 * 1024) {
+        int e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = min(max(A.ids[min(i0 + j * 1024, A.npairs - 1)], 0), A.E - 1) - e0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if ((unsigned)e[j] < (unsigned)kScaleExperts) used[e[j]] = 1;
+    }
+    __syncthreads();
+    // 8 values per thread; suh_u follows suh_g
+    const int n = 2 * A.g.H;
+    for (int i = t * 8; i < kScaleExperts * n; i += 8 * 1024) {
+        const int e = i / n, c = i % n;
+        if (used[e]) *(half8_t*)(A.suh + (size_t)e0 * n + i) = ld_half8((const uint8_t*)A.ptrs[e0 + e] + A.g.off_suh_g + 2 * c);
+    }
+}
+
 // ---- input Hadamards ---------------------------------------------------------------------------------------------------
 // xh[pick][pj][kb * 128 ..] = fp16(H(fp16(x[row] suh_pj)) / sqrt 128), one wave per (4 picks, kbs 128-blocks) and both
 // projections: 16 lanes hold a pick's block, 8 values each (row_fwht128_signed). Few registers, no LDS, full cache lines
@@ -126,7 +156,9 @@ __device__ __forceinline__ void xh_task(const GroupedArgs& A, int task, int kbs)
     const int ks = task % nks, p = task / nks * 4 + (l >> 4), c = (l & 15) * 8;
     const int s = min(p, A.npairs - 1);          // (lanes past the end repeat the last pick and store nothing)
     const size_t xo = (size_t)(s / A.topk) * A.x_stride + c;
-    const uint8_t* su = (const uint8_t*)A.ptrs[min(max(A.ids[s], 0), A.E - 1)] + A.g.off_suh_g + 2 * c;
+    const int e = min(max(A.ids[s], 0), A.E - 1);
+    const uint8_t* su = A.suh ? (const uint8_t*)(A.suh + (size_t)e * 2 * H + c)
+                              : (const uint8_t*)A.ptrs[e] + A.g.off_suh_g + 2 * c;
     half_t* o = A.xh + (size_t)s * 2 * H + c;
     const float rs = row_sign() * kRsqrt128;
     const int kb1 = min(nkb, (ks + 1) * kbs);
@@ -234,10 +266,14 @@ static int pass_rows(int M, int topk, int H, int I) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(M, np / topk));
 }
 
+// (up to 16 picks per expert the scales are at most 5 % of what an expert's products read; the workspace has room for
+// min(E, np / 16) experts' scales, which grows with both)
+static bool grouped_scales(size_t np, int E) { return np > (size_t)16 * E; }
+
 size_t grouped_workspace_bytes(int M, int topk, int H, int I, int E, bool y32) {
     const size_t np = (size_t)pass_rows(M, topk, H, I) * topk;
     return align256((3 * grouped_max_items(np, E) + 2) * 4) + align256(np * 4) + align256(np * 4 * H) + align256(np * 2 * I) +
-           align256(np * H * (y32 ? 4 : 2));
+           align256(np * H * (y32 ? 4 : 2)) + align256(std::min<size_t>(E, np / 16) * 4 * H);
 }
 
 static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) {
@@ -257,6 +293,11 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
     a.xh = (half_t*)take(np * 4 * a.g.H);
     a.abuf = (half_t*)take(np * 2 * a.g.I);
     a.y = take(np * a.g.H * (y32 ? 4 : 2));
+    a.suh = nullptr;
+    if (grouped_scales(np, a.E)) {
+        a.suh = (half_t*)take((size_t)a.E * 4 * a.g.H);
+        hipLaunchKernelGGL(grouped_scales_kernel, dim3((unsigned)((a.E + kScaleExperts - 1) / kScaleExperts)), dim3(1024), 0, s, a);
+    }
     const int nkb = a.g.H / 128, nq = (a.npairs + 3) / 4;
     // 128-blocks per wave: one while the waves do not fill the chip several times over, then up to 4, which hides a
     // wave's own table lookups (8,192 tokens: 1 / 2 / 4 / 8 blocks 230 / 207 / 201 / 207 us; 16 rows: 5.4 / 5.6 / 8.6 us)

@@ -221,7 +221,13 @@ __device__ __forceinline__ void down_rows(const GroupedArgs& A, int e, int s0, i
         }
         regb_core<K, NB, false, 2>(rw, woff, tiles_n, ra, aoff, 0, I / 64, acc);
     }
-    // 16 rows per round, 16 lanes per (row, 128 columns), two units per thread
+    // 16 rows per round, 16 lanes per (row, 128 columns), two units per thread. The output scales are loaded once: per
+    // round, the 16 rows of an expert in host memory read as many bytes of them over PCIe as 40 % of its trellis
+    half8_u hs[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        hs[i] = ld_half8(base + A.g.off_svh_d +
+                         2 * (nt * 64 * WV + (((int)(threadIdx.x >> 4) + i * 4 * WV) >> 4) * 128 + (l & 15) * 8));
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         float* ep = (float*)lds + (b & 1) * 16 * kEpRowW<WV>;
@@ -231,14 +237,13 @@ __device__ __forceinline__ void down_rows(const GroupedArgs& A, int e, int s0, i
         for (int i = 0; i < 2; ++i) {
             const int un = (threadIdx.x >> 4) + i * 4 * WV, rr = un & 15, cb = (un >> 4) * 128 + (l & 15) * 8;
             const int row = 16 * b + rr, ch = nt * 64 * WV + cb;
-            const half8_u hs = ld_half8(base + A.g.off_svh_d + 2 * ch);
             const int pk = A.perm[s0 + min(row, rows - 1)];
             const float pw = A.w[pk];
             float v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = ep[rr * kEpRowW<WV> + cb + j];
             row_fwht128_signed(v);
-            if (row < rows) st_y<TY>(A.y, (size_t)pk * H + ch, v, row_sign() * kRsqrt128 * pw, hs);
+            if (row < rows) st_y<TY>(A.y, (size_t)pk * H + ch, v, row_sign() * kRsqrt128 * pw, hs[i]);
         }
     }
 }

@@ -93,3 +93,29 @@ def test_grouped_decode_sizes_any_alignment(K):
     r = _rel(got.float().cpu().numpy(), of)
     print(f"grouped decode sizes K={K}: rel-L2 fp16 {r:.2e}")
     assert r <= TOL
+
+
+def test_grouped_scales_only_of_the_experts_in_use():
+    """Above 16 picks per expert the input scales are copied first, of the experts that have picks: those without may have
+    no blob. 11 experts, three of them unused with a null entry, one pick for the last; results as with the blobs in place
+    in every entry and as with host-resident blobs."""
+    H, I, K, seed = 512, 256, 3, 9400
+    counts = [40, 0, 17, 64, 0, 100, 0, 30, 1, 20, 1]
+    print("case grouped scales", flush=True)
+    E, ids = len(counts), _ids_of(counts, seed)
+    M = ids.shape[0]
+    assert M > 16 * E
+    blobs = np.stack([synth.expert_blob(seed, e, H, I, K) for e in range(E)])
+    dev, host = torch.from_numpy(blobs).cuda(), torch.from_numpy(blobs).pin_memory()
+    full = torch.tensor([dev[e].data_ptr() for e in range(E)], dtype=torch.int64)
+    some = torch.where(torch.tensor(counts) > 0, full, torch.zeros_like(full))
+    pinned = torch.tensor([host[e].data_ptr() if counts[e] else 0 for e in range(E)], dtype=torch.int64)
+    x = torch.from_numpy(exl3.bf16_to_f32(synth.activations(seed, M, H))).cuda()
+    it, wt = torch.from_numpy(ids).cuda(), torch.ones(M, 1, device="cuda")
+    _ops().moe_set_prefill_min_m(1)
+    try:
+        a, b, c = (_ops().moe_forward(x, it, wt, t.cuda(), I, K, E) for t in (full, some, pinned))
+        torch.cuda.synchronize()
+    finally:
+        _ops().moe_set_prefill_min_m(256)
+    assert torch.equal(a, b) and torch.equal(a, c)
