@@ -271,8 +271,8 @@ def run_linear(args, dev):
     groups 2048 -> 12,288 of 4 shards, 4096 -> 2048, 2048 -> 1024 of 2 shards and 512 -> 2048; EXL3 K=3 mul1 unless
     --linear-k / --linear-cb say otherwise, seeded random trellis, bs=1 bf16 activations): 192 calls per token captured in one HIP graph and timed with HIP events around its
     replays. value = tokens per second of those calls; roofline = trellis bytes per token / time per token against the
-    8 TB/s HBM peak (each call's three kernels included). The same groups at 1,024 rows (the reconstruct + fp16 GEMM
-    path) give the prefill figure. cpu_baseline: oracle/cpu_path.CpuLinear (decode through the codebook table on every
+    8 TB/s HBM peak (each call's three kernels included). The same groups at 1,024 rows (the trellis decoded
+    inside an fp16 MFMA product) give the prefill figure. cpu_baseline: oracle/cpu_path.CpuLinear (decode through the codebook table on every
     call, fp32 matmuls) on one layer's groups at bs=1 on this host's cores, x 48 layers."""
     import numpy as np
     import torch
@@ -355,7 +355,7 @@ def run_linear(args, dev):
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK, 4), "traffic": None},
         "prefill_1024_rows": {"ms_per_layer": round(t_pf * 1e3, 4), "tflops": round(flops / t_pf / 1e12, 1),
-                              "route": "w8a8 int8 GEMM" if q8 else "fp16 GEMM",
+                              "route": "w8a8 int8 GEMM" if q8 else "trellis decoded into fp16 MFMA",
                               ("frac_int8_mfma" if q8 else "frac_fp16_mfma"): round(flops / t_pf / 1e12 / mm_peak, 4)},
     }
     log(f"dense linear: {t_tok * 1e6:.1f} us per token ({t_tok * 1e6 / (L * len(LINEAR_GROUPS)):.2f} us per call), "

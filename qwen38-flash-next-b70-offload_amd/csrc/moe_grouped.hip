@@ -16,8 +16,8 @@
 // takes 150-170 us and down 85-98 us, 89 % and 79 % of their VALU cycles issuing. Columns are split over waves, not K,
 // so that a weight is decoded by one wave and multiplied into every row, and nothing is exchanged before the epilogue.
 // Whole layers, bf16, before (one decode per pick, or a core that decodes into LDS for 192-row passes) and now:
-// 16 Zipf rows 104 -> 74 us, 64 rows 398 -> 132 us, 301 tokens 605 -> 240 us, 2,048 tokens 726 -> 402 us, 8,192 tokens
-// 1,290 -> 1,185 us; H 4096 / I 1536, 128 experts, top-8, K 2, 777 tokens: 861 -> 533 us.
+// 16 Zipf rows 104 -> 63 us, 64 rows 399 -> 120 us, 301 tokens 605 -> 232 us, 2,048 tokens 726 -> 363 us, 8,192 tokens
+// 1,269 -> 1,072 us; H 4096 / I 1536, 128 experts, top-8, K 2, 777 tokens: 861 -> 465 us.
 #include "exl3_common.cuh"
 #include "exl3_geom.h"
 #include "exl3_kernels.h"
