@@ -269,7 +269,8 @@ int exl3_linear_small(const void* x, int x_dtype, int64_t x_stride, int M, int k
 /* The same linear for any number of rows, with the input Hadamards, the trellis decode and the products in kernels of
  * its own (exl3_ops.sycl:651-757, the path above the fused rows). group_bounds: host [S + 1], shard g's columns
  * [group_bounds[g], group_bounds[g + 1]), multiples of width (256 or 128). S at most 16. The workspace (device, exl3_linear_rows_workspace bytes, no state between calls) holds the input
- * Hadamards and the partial sums. EXL3_EUNSUPPORTED if S M k fp16 values or the trellis reach 2 GiB. */
+ * Hadamards and the partial sums; its size is 0 for sizes that the call refuses (k not a multiple of 128, n not of width).
+ * EXL3_EUNSUPPORTED if S M k fp16 values or the trellis reach 2 GiB. */
 size_t exl3_linear_rows_workspace(int M, int k, int n, int S, int width);
 int exl3_linear_rows(const void* x, int x_dtype, int64_t x_stride, int M, int k, int n, const void* trellis, int K,
                      int cb, const void* suh, int S, const void* svh, const int64_t* group_bounds, int width, void* out,

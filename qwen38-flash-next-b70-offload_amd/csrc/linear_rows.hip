@@ -55,13 +55,15 @@ __global__ void __launch_bounds__(64 * kLxWaves) lin_xh_kernel(LinearArgs A) {
 
 // ---- host --------------------------------------------------------------------------------------------------------------
 
+// (M > 0, n a positive multiple of width)
 int linear_rows_slices(int M, int k, int n, int width) {
-    const int rt = 16 * linear_rows_blocks(M), wgs = (n / width) * ((M + rt - 1) / rt), nkb = k / 128;
+    const int64_t rt = 16 * linear_rows_blocks(M), wgs = n / width * ((M + rt - 1) / rt);
+    const int nkb = k / 128;
     // about one workgroup of 8 waves per CU: more slices cost their partial sums' traffic (40 rows, 2048 -> 12,288, K 4,
     // 48 workgroups: 1 / 2 / 4 / 8 slices 37 / 29 / 26 / 34 us; 1,024 rows, 4096 -> 2048, 64 workgroups: 84 / 58 / 48 /
     // 61 us), and up to 512 input rows a second launch for the sums costs more than the slices give (1,024 rows, 512 ->
     // 2048: 25 against 31 us)
-    return nkb <= 4 ? 1 : std::max(1, std::min(std::min(8, nkb / 2), 256 / wgs));
+    return nkb <= 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(std::min(8, nkb / 2), 256 / wgs));
 }
 
 hipError_t launch_linear_rows(int K, int cb, const LinearRowsArgs& a, int width, float* part, void* out, int out_dt,

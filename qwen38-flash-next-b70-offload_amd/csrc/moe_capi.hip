@@ -1017,7 +1017,8 @@ int exl3_linear_small(const void* x, int x_dtype, int64_t x_stride, int M, int k
 // the workspace of a linear_rows call: xh [S][M][k] fp16, then the partial sums [P][M][n] fp32 of its K-slices
 static size_t linear_rows_xh_bytes(int M, int k, int S) { return align256((size_t)S * M * k * 2); }
 size_t exl3_linear_rows_workspace(int M, int k, int n, int S, int width) {
-    if (M <= 0 || k <= 0 || n <= 0 || S <= 0 || (width != 128 && width != 256)) return 0;
+    // sizes that exl3_linear_rows refuses need none (a caller asks for the size before the call)
+    if (M <= 0 || k <= 0 || n <= 0 || S <= 0 || (width != 128 && width != 256) || k % 128 || n % width) return 0;
     const int P = linear_rows_slices(M, k, n, width);
     return linear_rows_xh_bytes(M, k, S) + (P > 1 ? align256((size_t)P * M * n * 4) : 0);
 }

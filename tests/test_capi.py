@@ -1,6 +1,9 @@
 """C-ABI library: loads, exports every function include/exl3moe.h declares, validates arguments on the host (no
 compute calls: this runs without a GPU)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -76,3 +79,18 @@ def test_linear_entry_points_validate_without_a_gpu():
     assert L.exl3_reconstruct(None, 128, 256, 16, 8, 3, 2, None, None) == 1
     assert L.exl3_had_in(None, 0, 0, 0, 256, None, 1, None, None) == 0
     assert L.exl3_had_out(None, 1, 100, None, None, 0, 100, None) == 1
+
+
+@pytest.mark.parametrize("M,k,n,S,width,some", [(9, 2048, 128, 1, 256, False), (9, 2048, 384, 1, 256, False),
+                                                (9, 100, 256, 1, 256, False), (9, 64, 128, 1, 128, False),
+                                                (9, 2048, 128, 1, 128, True), (1, 128, 256, 1, 256, True),
+                                                (40, 2048, 12288, 4, 256, True), (1 << 22, 1024, 1 << 26, 1, 128, True),
+                                                ((1 << 31) - 1, 128, 256, 1, 256, True)])
+def test_linear_rows_workspace_of_any_sizes(M, k, n, S, width, some):
+    """The size query answers whatever its arguments (in a process of its own, which a division by zero would end): 0
+    for sizes that exl3_linear_rows refuses, else at least the fp16 input Hadamards."""
+    r = subprocess.run([sys.executable, "-c", f"from exl3xpu import capi; "
+                        f"print(capi.lib().exl3_linear_rows_workspace({M}, {k}, {n}, {S}, {width}))"],
+                       env={**os.environ, "PYTHONPATH": os.pathsep.join(sys.path)}, capture_output=True, text=True)
+    assert r.returncode == 0, (r.returncode, r.stderr[-300:])
+    assert int(r.stdout) >= 2 * S * M * k if some else int(r.stdout) == 0
