@@ -101,11 +101,12 @@ int exl3_set_decision_log(int32_t* buf, int64_t cap_words);
 
 /* workspace bytes of an exl3_moe_forward call with these sizes (small decode calls: the blob pointer of every pick; the
  * grouped kernels otherwise: sorted routing, input Hadamards [M topk][2][H] fp16, abuf [M topk][I] fp16, y [M topk][H]
- * fp16, or fp32 below prefill_min_m; calls of more picks than one pass takes share the workspace of a pass). The decode kernel's cross-workgroup exchange is not in the workspace: the
- * library owns one zeroed device buffer per device and grows it when a call needs more (hipMalloc + hipMemset, after
- * a device synchronisation; the replaced buffer stays allocated, since graphs captured earlier still address it); a
- * call that would grow it while its stream is being captured fails with EXL3_EUNSUPPORTED, so run one call of the
- * largest size before capturing. */
+ * fp16, or fp32 below prefill_min_m; calls of more picks than one pass takes share the workspace of a pass). It never
+ * falls as M grows, so the size for a caller's largest M serves its smaller calls. The decode kernel's cross-workgroup
+ * exchange is not in the workspace: the library owns one zeroed device buffer per device and grows it when a call needs
+ * more (hipMalloc + hipMemset, after a device synchronisation; the replaced buffer stays allocated, since graphs captured
+ * earlier still address it); a call that would grow it while its stream is being captured fails with EXL3_EUNSUPPORTED,
+ * so run one call of the largest size before capturing. */
 size_t exl3_moe_forward_workspace(int M, int H, int I, int topk, int n_experts);
 
 /* moe_forward (a8:1221-1225 -> moe_forward_impl a8:1263-1314): out[m] = sum_k w[m,k] * expert(ids[m,k])(x[m]).

@@ -273,8 +273,12 @@ static bool grouped_y32(int M, int topk) { return !use_prefill(M, topk); }
 size_t exl3_moe_forward_workspace(int M, int H, int I, int topk, int n_experts) {
     if (M <= 0 || topk <= 0 || H <= 0 || I <= 0) return 0;
     const int E = std::min(std::max(n_experts, 1), kMaxExperts);
-    if (use_grouped(M, topk, H, I)) return grouped_workspace_bytes(M, topk, H, I, E, grouped_y32(M, topk));
-    return decode_workspace_bytes(M * topk, H, I);
+    if (!use_grouped(M, topk, H, I)) return decode_workspace_bytes(M * topk, H, I);
+    // the pick outputs become fp16 above the decode sizes (H 2048, I 512, top-10: 102 rows need 18.3 MB, 103 rows 14.2 MB):
+    // the size covers the decode-size calls of as many picks too, so that it never falls as the rows grow
+    const int few = (int)std::min<int64_t>((int64_t)M * topk, kMaxPairs);
+    return std::max(grouped_workspace_bytes(M, topk, H, I, E, grouped_y32(M, topk)),
+                    grouped_workspace_bytes(1, few, H, I, E, true));
 }
 
 static int64_t* pair_ptr_area(void* ws, int npairs, int H, int I) {

@@ -44,6 +44,20 @@ def test_forward_rejects_bad_dtype_and_workspace():
     assert L.exl3_moe_align_workspace(8192, 10, 512) == 80 * 512 * 4
 
 
+@pytest.mark.parametrize("H,I,E,topk", [(2048, 512, 512, 10), (4096, 1536, 128, 8), (2048, 512, 32, 10), (512, 256, 8, 3),
+                                        (4096, 1536, 128, 1)])
+@pytest.mark.parametrize("min_m", [1, 64, 256])
+def test_forward_workspace_never_falls_as_the_rows_grow(H, I, E, topk, min_m):  # noqa: E741
+    """A caller sizes one workspace for its largest batch and runs smaller ones in it."""
+    L = capi.lib()
+    assert L.exl3_set_prefill_min_m(min_m) == 0
+    try:
+        b = [L.exl3_moe_forward_workspace(M, H, I, topk, E) for M in [*range(1, 1200), 4096, 8192, 60000]]
+    finally:
+        L.exl3_set_prefill_min_m(256)
+    assert all(x <= y for x, y in zip(b, b[1:])), [i + 1 for i in range(len(b) - 1) if b[i] > b[i + 1]][:4]
+
+
 def test_setters():
     L = capi.lib()
     assert L.exl3_set_host_stride(7) == 1
