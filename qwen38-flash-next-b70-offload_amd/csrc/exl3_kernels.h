@@ -91,7 +91,16 @@ struct AlignOut {
     int* pair_tok; int* pair_of; float* pair_w;                                    // [npairs] each
 };
 
-// picks grouped by expert, few rows each (moe_grouped.hip)
+// the misses of a cached call, as its ensure left them (exl3_fill.cuh)
+struct FillArgs {
+    const int32_t* list;                           // [1 + n] their count and experts; null: no cached call
+    int64_t* ptrs; int64_t* fill;                  // the layer's tables [E]: blob address, address of the new slot (or 0)
+    const int32_t* vict; const int64_t* vaddr;     // victim list or null, write-back targets or null (EnsureArgs)
+    const int64_t* host_base; int64_t hstride;     // write-back target without vaddr
+    int64_t sstride; uint8_t* ram_res;             // bytes of a slot; residency flags of the keys or null
+};
+
+// picks grouped by expert (moe_grouped.hip)
 struct GroupedArgs {
     const void* x; int x_dt; int64_t x_stride;     // activations [M, H]
     const int32_t* ids; const float* w;            // [M * topk]
@@ -99,7 +108,8 @@ struct GroupedArgs {
     const int64_t* ptrs;                           // per-layer blob pointer table [E]
     int* perm;                                     // pick at every sorted position [npairs]
     int rmax;                                      // rows of an item at most (64 or 192)
-    int* it_expert; int* it_start; int* it_cnt;    // items: up to rmax sorted positions of one expert, longest first
+    int64_t* it_blob; int* it_start; int* it_cnt;  // items: up to rmax sorted positions of one expert (its blob), longest
+                                                   // first
     int* n_items;                                  // [2] items, and those of more than 16 rows (the first ones)
     _Float16* suh;                                 // [E][2][H] input scales of the experts in use, or null: in the blobs
     _Float16* xh;                                  // [npairs][2][H] input Hadamards (gate, up)
@@ -107,6 +117,7 @@ struct GroupedArgs {
     void* y;                                       // [npairs][H] fp32 or fp16, routing weight applied
     void* out; int64_t out_stride;                 // [M, H], dtype of x
     BlobGeom g;
+    FillArgs f;
 };
 
 constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -177,9 +188,6 @@ hipError_t launch_ensure(const EnsureArgs& a, hipStream_t s);
 // prefetch (moe_prefetch a8:1194-1222): ensure in prefetch mode, then copy every assigned expert from its host record
 // (host_base[layer] + e * hstride) into its slot (slot_base + s * sstride, `copy_bytes` bytes) and repoint ptrs_all
 hipError_t launch_prefetch(const EnsureArgs& a, int64_t sstride, int64_t copy_bytes, hipStream_t s);
-// the copies and the commit of a cached call outside the decode kernel, after its ensure (a: the ensure's arguments;
-// blob: bytes of the layer's blob; max_n: an upper bound of the call's fills)
-hipError_t launch_cached_fills(const EnsureArgs& a, int64_t blob, int max_n, uint8_t* ram_res, hipStream_t s);
 hipError_t launch_scatter_flags(uint8_t* flags, int64_t n_flags, const int32_t* packed, int64_t n, hipStream_t s);
 hipError_t launch_table_update(int64_t* ptrs_all, int32_t* slot_of, int32_t* slot_key, int32_t* slot_last,
                                const int64_t* rec, int64_t n, hipStream_t s);
@@ -195,7 +203,7 @@ struct TierPool {
 };
 hipError_t launch_tier_exchange(uint8_t* flags, int64_t n_flags, const int32_t* packed, int64_t n_diff,
                                 const TierRing& rg, const TierCopies& cp, const TierPool& pl, hipStream_t s);
-// prefill.hip
+// align.hip
 hipError_t launch_align(const int32_t* ids, const float* w, int npairs, int topk, int E, int pad, int* chunk_scratch,
                         const AlignOut& o, hipStream_t s);
 size_t align_scratch_bytes(int npairs, int E);

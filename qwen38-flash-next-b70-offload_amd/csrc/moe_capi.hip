@@ -252,9 +252,9 @@ int exl3_set_decision_log(int32_t* buf, int64_t cap_words) {
     return EXL3_OK;
 }
 
-// the prefill kernels serve a call from prefill_min_m rows on, and also below it when the call has more picks or rows
-// than the fused decode kernel takes (the reference's align path covers pair_max_m < M < prefill_min_m, a8:1277-1314;
-// the prefill kernels here are exact from M = 1 on)
+// a call of the prefill sizes (16-bit pick outputs, as the reference's prefill keeps them): from prefill_min_m rows on, and
+// below that with more picks or rows than the fused decode kernel takes (the reference's align path covers pair_max_m < M <
+// prefill_min_m, a8:1277-1314)
 static bool exceeds_decode(int M, int topk) { return (int64_t)M * topk > kMaxPairs || M > kMaxRows; }
 static bool use_prefill(int M, int topk) { return M >= g_cfg.prefill_min_m || exceeds_decode(M, topk); }
 
@@ -263,6 +263,9 @@ static bool use_prefill(int M, int topk) { return M >= g_cfg.prefill_min_m || ex
 // experts of I >= 1024). Below that the fused kernel's single launch is faster, or the experts' workgroups divide badly
 // over the CUs: at H 2048 / I 512, top-10, 54 us against 67 us for 8 rows of distinct experts (80 picks), but 79 against
 // 56 us for 12 Zipf rows; at H 4096 / I 1536, top-8, K 4, 97 against 109 us for 3 rows and 126 against 110 us for 4.
+// Cached calls cross at the same sizes, with hits only and with misses: H 2048 / I 512, 11 rows, 100 / 99 / 95 / 90 % of
+// the experts in slots 88 / 99 / 175 / 301 against 61 / 98 / 175-179 / 288-295 us; H 4096 / I 1536, K 2, 4 rows
+// 128 / 147 / 235 / 364 against 112 / 134 / 229-234 / 354-366, K 3 133 / 168 / 329 / 542 against 113 / 146 / 292-302 / 487-502.
 static bool use_grouped(int M, int topk, int H, int I) {
     const int64_t min_work = I >= 1024 ? 49000 : 56000;
     return H % 256 == 0 && (use_prefill(M, topk) || (int64_t)M * topk * I >= min_work);
@@ -339,7 +342,7 @@ static int forward_impl(const void* x, int x_dtype, int64_t x_stride, int M, int
                         size_t ws_bytes, hipStream_t st, const int64_t* fill, int64_t* commit_ptrs, int64_t* commit_fill,
                         const int32_t* fill_list, const int64_t* pair_ptr, const VictimArgs* va = nullptr,
                         int max_victims = 0, const EnsureArgs* fused_ens = nullptr, bool vict_inline = false,
-                        uint64_t* xb_given = nullptr) {
+                        uint64_t* xb_given = nullptr, const FillArgs* fills = nullptr) {
     if (!fill && use_prefill(M, topk)) {
         if (H % 256) return fail(EXL3_EUNSUPPORTED, "moe prefill: H %% 256 == 0 required (H=%d)", H);
         if ((int64_t)M * topk > (1 << 28)) return fail(EXL3_EUNSUPPORTED, "moe prefill: %d x %d pairs", M, topk);
@@ -362,6 +365,7 @@ static int forward_impl(const void* x, int x_dtype, int64_t x_stride, int M, int
         ga.out = out;
         ga.out_stride = out_stride;
         ga.g = blob_geom(H, I, K);
+        if (fills) ga.f = *fills;
         const hipError_t e = launch_grouped(ga, y32, ws, st);
         return e == hipSuccess ? EXL3_OK : hip_fail(e, "moe grouped launch");
     }
@@ -617,7 +621,7 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
     const int P = M * topk;
     const bool grouped = exceeds_decode(M, topk) || use_grouped(M, topk, H, I);
     if (exceeds_decode(M, topk) && xb)
-        return fail(EXL3_EUNSUPPORTED, "moe_forward_cached_static: %d x %d picks take the prefill kernels, which need "
+        return fail(EXL3_EUNSUPPORTED, "moe_forward_cached_static: %d x %d picks are a prefill-size call, which needs "
                     "a workspace (use exl3_moe_forward_cached)", M, topk);
     EnsureArgs ea{};
     ea.ids = topk_ids;
@@ -670,9 +674,9 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
     ea.log = g_cfg.log;
     ea.log_cap = g_cfg.log_cap;
     if (grouped) {
-        // one ensure over all the picks, victim write-back, fill copies and the commit, then the grouped kernels over
-        // the committed table (the caller's ids and w carry the tier mask)
-        if (H % 256) return fail(EXL3_EUNSUPPORTED, "moe_forward_cached: %d picks need the prefill kernels (H %% 256)", P);
+        // one ensure over all the picks, then the grouped kernels, which copy the misses into their slots, write the
+        // victims back and commit the table beside their own work (the caller's ids and w carry the tier mask)
+        if (H % 256) return fail(EXL3_EUNSUPPORTED, "moe_forward_cached: %d picks need the grouped kernels (H %% 256)", P);
         const size_t need = grouped_workspace_bytes(M, topk, H, I, E, grouped_y32(M, topk));
         if (!workspace || workspace_bytes < need)
             return fail(EXL3_EWORKSPACE, "moe_forward_cached: workspace %zu < %zu bytes", workspace_bytes, need);
@@ -682,10 +686,21 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
         hipError_t e = launch_ensure(ea, st);
         if (e == hipErrorInvalidValue) return fail(EXL3_EUNSUPPORTED, "moe_forward_cached: ensure state does not fit in LDS");
         if (e != hipSuccess) return hip_fail(e, "ensure launch");
-        e = launch_cached_fills(ea, g.blob, std::min(std::min(ea.max_fill, E), P), vict_res, st);
-        if (e != hipSuccess) return hip_fail(e, "cached fills launch");
+        FillArgs f{};
+        if (ea.max_fill > 0) {
+            f.list = fill_list;
+            f.ptrs = ptrs_all + (int64_t)layer * E;
+            f.fill = fill_all + (int64_t)layer * E;
+            f.vict = ea.vict;
+            f.vaddr = ea.vict_addr;
+            f.host_base = host_base;
+            f.hstride = ea.hstride;
+            f.sstride = ea.blob;
+            f.ram_res = vict_res;
+        }
         return forward_impl(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs_all + (int64_t)layer * E, I, K, E,
-                            out, out_stride, workspace, workspace_bytes, st, nullptr, nullptr, nullptr, nullptr, nullptr);
+                            out, out_stride, workspace, workspace_bytes, st, nullptr, nullptr, nullptr, nullptr, nullptr,
+                            nullptr, 0, nullptr, false, nullptr, &f);
     }
     const size_t need = decode_workspace_bytes(P, H, I);
     if (!workspace || workspace_bytes < need)
@@ -742,8 +757,9 @@ static_assert(decode_workspace_bytes(kMaxPairs, 0, 0) <= kStaticPtrBytes,
 static_assert(kStaticPtrBytes % 256 == 0 && kStaticPtrBytes < kStaticScratchBytes, "static scratch layout");
 static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
 // the grouped kernels' workspace of a static call, in an array of its own (its data could pass as a tag): per pick it
-// takes 8 H + 2 I bytes where the exchange words take at least 16 I + 8 H, so every call that the exchange words admit
-// fits beside the sort's lists
+// takes 8 H + 2 I bytes and at most H / 4 more for the copied input scales, where the exchange words take at least 16 I +
+// 8 H. The exchange words admit 8 H picks <= 8 MiB and a grouped call has I picks >= 49,000, so H / 4 < 14 I: every call
+// that they admit fits beside the sort's lists
 constexpr size_t kStaticGroupedBytes = kStaticScratchBytes + (64 << 10);
 static __device__ __align__(256) uint8_t grouped_scratch[kStaticGroupedBytes];
 static std::mutex g_scratch_mu;

@@ -8,6 +8,7 @@
 //            by pick; epilogue through LDS: g/u Hadamards, SwiGLU, * suh_d, Hadamard -> abuf[pick] (fp16)
 //   down     per (item, 64 WV columns of H), K = I, the same core; output Hadamard * (w * svh_d) -> y[pick]
 //   combine  out[m] = sum over the row's picks of y, in pick order (fp32)
+// A cached call's misses are copied into their slots by workgroups of the same launches (FILL, exl3_fill.cuh).
 // (reference: kernels/moe-a8/exl3_moe.a8.sycl:121-395, 422-635, 639-680, with the same fp16 rounding points.)
 //
 // What bounds them: the decode's VALU work, 3.5 instructions per weight (bfe, mul_lo, sad, half a pk_fma) at 4.2 to 4.6
@@ -19,6 +20,7 @@
 // 16 Zipf rows 104 -> 63 us, 64 rows 399 -> 120 us, 301 tokens 605 -> 232 us, 2,048 tokens 726 -> 363 us, 8,192 tokens
 // 1,269 -> 1,072 us; H 4096 / I 1536, 128 experts, top-8, K 2, 777 tokens: 861 -> 465 us.
 #include "exl3_common.cuh"
+#include "exl3_fill.cuh"
 #include "exl3_geom.h"
 #include "exl3_kernels.h"
 #include "exl3_regb.cuh"
@@ -63,10 +65,14 @@ __device__ __forceinline__ uint64_t block_scan64(uint64_t v, uint64_t* sw, uint6
 // thread e: the items of expert e (tot rows from sorted position st): the fewest items of at most rmax rows, cut evenly
 // in 16-row blocks; ordered by descending block count over all experts (packed scans of 16 bits per block count), so
 // that the longest start first. n_items[0]: all items, [1]: those of more than one block.
-constexpr int kMaxBlocks = 12;
 __device__ __forceinline__ void emit_items(const GroupedArgs& A, int e, int st, int tot, uint64_t* sw) {
     const int n = (tot + A.rmax - 1) / A.rmax, nb = n ? ((tot + n - 1) / n + 15) >> 4 : 0;   // items, blocks of each
     int above = 0;
+    int64_t blob = 0;
+    if (n) {                                     // (a miss of a cached call: its new slot)
+        blob = A.ptrs[e];
+        if (A.f.list && A.f.fill[e]) blob = A.f.fill[e];
+    }
     for (int g = (A.rmax + 63) / 64 - 1; g >= 0; --g) {          // block counts 4 g + 1 .. 4 g + 4
         uint64_t tt;
         const uint64_t ex = block_scan64(nb > 4 * g && nb <= 4 * g + 4 ? (uint64_t)n << (16 * (nb - 1 - 4 * g)) : 0ull, sw, tt);
@@ -75,7 +81,7 @@ __device__ __forceinline__ void emit_items(const GroupedArgs& A, int e, int st, 
             if (4 * g + k == nb) {
                 int p = above + (int)((ex >> (16 * (k - 1))) & 0xFFFF);
                 for (int i = 0; i < n; ++i, ++p) {
-                    A.it_expert[p] = e;
+                    A.it_blob[p] = blob;
                     A.it_start[p] = st + i * 16 * nb;
                     A.it_cnt[p] = min(16 * nb, tot - i * 16 * nb);
                 }
@@ -119,8 +125,9 @@ __device__ __forceinline__ void sort_wg(const GroupedArgs& A, int* off /* LDS [E
 // The input Hadamards run in pick order and read an expert's input scales for each of its picks: 8 KB per pick and expert
 // of H 2048. That is cache traffic for an expert in HBM, but host memory is not cached, so with a third of 512 experts
 // read over PCIe and 160 picks per expert it was 230 MB next to the 412 MB of their records (8,192 tokens 12.7 ms per
-// layer, 8.2 ms with the copies and with down's output scales loaded once; with every expert in HBM 1.09 ms either way). So each expert's scales are copied once: a workgroup per kScaleExperts experts looks for
-// them in the ids (an expert without picks may have no blob) and copies those that it finds.
+// layer, 8.2 ms with the copies and with down's output scales loaded once; with every expert in HBM 1.09 ms either way).
+// So each expert's scales are copied once: a workgroup per kScaleExperts experts looks for them in the ids (an expert
+// without picks may have no blob) and copies those that it finds.
 constexpr int kScaleExperts = 4;
 __global__ void __launch_bounds__(1024) grouped_scales_kernel(GroupedArgs A) {
     __shared__ int used[kScaleExperts];
@@ -193,6 +200,7 @@ __device__ __forceinline__ void xh_task(const GroupedArgs& A, int task, int kbs)
     }
 }
 
+template <bool FILL>
 __global__ void __launch_bounds__(kPreThreads) __attribute__((amdgpu_waves_per_eu(8)))
 grouped_pre_kernel(GroupedArgs A, int ntask, int kbs) {
     __shared__ int off[kMaxExperts];
@@ -201,8 +209,17 @@ grouped_pre_kernel(GroupedArgs A, int ntask, int kbs) {
         sort_wg(A, off, sw);
         return;
     }
+    int blk = blockIdx.x - 1;
+    if constexpr (FILL) {                        // a cached call's misses: what gate/up reads of them
+        if (blk < fill_workgroups(kPreThreads)) {
+            fill_part<kPreThreads>(A, 0, blk);
+            if (A.rmax > 64) fill_part<kPreThreads>(A, 1, blk);   // (the large gate/up kernel copies nothing)
+            return;
+        }
+        blk -= fill_workgroups(kPreThreads);
+    }
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int task = (blockIdx.x - 1) * (kPreThreads / 64) + wv;
+    const int task = blk * (kPreThreads / 64) + wv;
     if (task >= ntask) return;                   // (whole waves: the transforms need every lane)
     if (A.x_dt == 1) xh_task<1>(A, task, kbs);
     else if (A.x_dt == 2) xh_task<2>(A, task, kbs);
@@ -212,10 +229,16 @@ grouped_pre_kernel(GroupedArgs A, int ntask, int kbs) {
 // out[m][h] = sum over the row's picks, in pick order, of y[m topk + k][h]; one thread per 8 columns. The picks' rows are
 // loaded kComb at a time before they are summed (picks past topk repeat the last one and are not summed).
 constexpr int kComb = 10;
-template <typename TY>
+template <typename TY, bool FILL>
 __global__ void __launch_bounds__(128) grouped_combine_kernel(GroupedArgs A) {
     const int H = A.g.H, topk = A.topk, m = blockIdx.x;
     const int h0 = (blockIdx.y * 128 + threadIdx.x) * 8;
+    if (FILL && blockIdx.x == 0 && blockIdx.y == 0)              // a cached call's misses are in their slots: commit them
+        for (int mi = threadIdx.x; mi < A.f.list[0]; mi += 128) {
+            const int e = A.f.list[1 + mi];
+            A.f.ptrs[e] = A.f.fill[e];
+            A.f.fill[e] = 0;
+        }
     if (h0 >= H) return;
     float acc[8] = {};
     for (int k0 = 0; k0 < topk; k0 += kComb) {
@@ -272,7 +295,7 @@ static bool grouped_scales(size_t np, int E) { return np > (size_t)16 * E; }
 
 size_t grouped_workspace_bytes(int M, int topk, int H, int I, int E, bool y32) {
     const size_t np = (size_t)pass_rows(M, topk, H, I) * topk;
-    return align256((3 * grouped_max_items(np, E) + 2) * 4) + align256(np * 4) + align256(np * 4 * H) + align256(np * 2 * I) +
+    return align256((4 * grouped_max_items(np, E) + 2) * 4) + align256(np * 4) + align256(np * 4 * H) + align256(np * 2 * I) +
            align256(np * H * (y32 ? 4 : 2)) + align256(std::min<size_t>(E, np / 16) * 4 * H);
 }
 
@@ -284,11 +307,11 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
     a.rmax = np > (size_t)56 * a.E && a.g.I % 256 == 0 && a.g.H % 512 == 0 && !y32 ? 192 : 64;
     uint8_t* p = (uint8_t*)ws;
     auto take = [&p](size_t n) { uint8_t* q = p; p += align256(n); return q; };
-    int* it = (int*)take((3 * mi + 2) * 4);
-    a.it_expert = it;
-    a.it_start = it + mi;
-    a.it_cnt = it + 2 * mi;
-    a.n_items = it + 3 * mi;
+    int* it = (int*)take((4 * mi + 2) * 4);
+    a.it_blob = (int64_t*)it;
+    a.it_start = it + 2 * mi;
+    a.it_cnt = it + 3 * mi;
+    a.n_items = it + 4 * mi;
     a.perm = (int*)take(np * 4);
     a.xh = (half_t*)take(np * 4 * a.g.H);
     a.abuf = (half_t*)take(np * 2 * a.g.I);
@@ -304,7 +327,10 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
     int kbs = 1;
     while (kbs < 4 && nq * ((nkb + kbs - 1) / kbs) > 32768) kbs *= 2;
     const int ntask = nq * ((nkb + kbs - 1) / kbs);
-    hipLaunchKernelGGL(grouped_pre_kernel, dim3(1 + (unsigned)((ntask + 15) / 16)), dim3(kPreThreads), 0, s, a, ntask, kbs);
+    const unsigned grid = 1 + (unsigned)((ntask + 15) / 16);
+    auto pre = [&](auto kern, unsigned n) { hipLaunchKernelGGL(kern, dim3(n), dim3(kPreThreads), 0, s, a, ntask, kbs); };
+    if (a.f.list) pre(grouped_pre_kernel<true>, fill_workgroups(kPreThreads) + grid);
+    else pre(grouped_pre_kernel<false>, grid);
     switch (a.g.K) {
         case 2: launch_products<2>(a, y32, s); break;
         case 3: launch_products<3>(a, y32, s); break;
@@ -312,8 +338,9 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
         default: return hipErrorInvalidValue;
     }
     const dim3 gc((unsigned)a.M, (unsigned)((a.g.H + 1023) / 1024));
-    if (y32) hipLaunchKernelGGL(grouped_combine_kernel<float>, gc, dim3(128), 0, s, a);
-    else hipLaunchKernelGGL(grouped_combine_kernel<half_t>, gc, dim3(128), 0, s, a);
+    auto combine = [&](auto kern) { hipLaunchKernelGGL(kern, gc, dim3(128), 0, s, a); };
+    if (a.f.list) combine(y32 ? grouped_combine_kernel<float, true> : grouped_combine_kernel<half_t, true>);
+    else combine(y32 ? grouped_combine_kernel<float, false> : grouped_combine_kernel<half_t, false>);
     return hipGetLastError();
 }
 
@@ -328,6 +355,7 @@ hipError_t launch_grouped(const GroupedArgs& a0, bool y32, void* ws, hipStream_t
         a.out = (uint8_t*)a0.out + (int64_t)m0 * a0.out_stride * esz;
         a.ids = a0.ids + (size_t)m0 * a.topk;
         a.w = a0.w + (size_t)m0 * a.topk;
+        if (m0) a.f = FillArgs{};                // (committed by the first pass)
         const hipError_t e = launch_pass(a, y32, ws, s);
         if (e != hipSuccess) return e;
     }

@@ -2,6 +2,7 @@
 // a translation unit of its own (moe_products_k2.hip, ...).
 #pragma once
 #include "exl3_common.cuh"
+#include "exl3_fill.cuh"
 #include "exl3_geom.h"
 #include "exl3_kernels.h"
 #include "exl3_regb.cuh"
@@ -20,8 +21,8 @@ constexpr int kEpRow = 260;                      // floats per row of the [16][2
 // wave-uniform values that the compiler loads per lane, as scalars: a descriptor in vector registers would make every
 // buffer load a loop over its lanes
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ const uint8_t* expert_base(const GroupedArgs& A, int e) {
-    const uint64_t p = (uint64_t)A.ptrs[e];
+__device__ __forceinline__ const uint8_t* item_blob(const GroupedArgs& A, int a) {
+    const uint64_t p = (uint64_t)A.it_blob[a];
     return (const uint8_t*)(((uint64_t)(uint32_t)uni((int)(p >> 32)) << 32) | (uint32_t)uni((int)p));
 }
 
@@ -65,12 +66,12 @@ __device__ __forceinline__ void st_y(void* y, size_t o, const float (&v)[8], flo
 
 // an item of one block: 4 waves of 64 columns (128 of I, both projections) in each of KS K-slices
 template <int K, int KS>
-__device__ __forceinline__ void gateup_item(const GroupedArgs& A, int e, int s0, int rows, int nb, float* ep) {
+__device__ __forceinline__ void gateup_item(const GroupedArgs& A, int a, int s0, int rows, int nb, float* ep) {
     constexpr int NB = 1;
     const int I = A.g.I, H = A.g.H, tiles_n = 2 * I / 16, l = lane_id();
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wc = wv & 3, ks = wv >> 2, pj = wc >> 1;
     using B = RegB<K, false, 2>;
-    const uint8_t* base = expert_base(A, e);
+    const uint8_t* base = item_blob(A, a);
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, (int)A.g.gu_bytes, 0x00020000);
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(A.xh, (short)0, A.npairs * 4 * H, 0x00020000);
     uint32_t aoff[NB];
@@ -132,13 +133,13 @@ __device__ __forceinline__ void gateup_item(const GroupedArgs& A, int e, int s0,
 template <int WV> constexpr int kEpRowW = 64 * WV + 4;
 
 template <int K, int NB, int WV>
-__device__ __forceinline__ void gateup_rows(const GroupedArgs& A, int e, int s0, int rows, int nb, uint8_t* lds) {
+__device__ __forceinline__ void gateup_rows(const GroupedArgs& A, int a, int s0, int rows, int nb, uint8_t* lds) {
     const int I = A.g.I, H = A.g.H, tiles_n = 2 * I / 16, l = lane_id();
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pj = wv / (WV / 2), wc = wv % (WV / 2);
     using B = RegB<K, false, 2>;
     using U = AUnits<NB, WV, 2>;
-    const uint8_t* base = expert_base(A, e);
+    const uint8_t* base = item_blob(A, a);
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, (int)A.g.gu_bytes, 0x00020000);
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(A.xh, (short)0, A.npairs * 4 * H, 0x00020000);
     uint32_t soff[U::NU];
@@ -191,12 +192,12 @@ __device__ __forceinline__ void gateup_rows(const GroupedArgs& A, int e, int s0,
 
 // (LDSA: A staged through LDS, else each wave's own loads)
 template <int K, int NB, int WV, bool LDSA, typename TY>
-__device__ __forceinline__ void down_rows(const GroupedArgs& A, int e, int s0, int rows, int nt, uint8_t* lds) {
+__device__ __forceinline__ void down_rows(const GroupedArgs& A, int a, int s0, int rows, int nt, uint8_t* lds) {
     const int I = A.g.I, H = A.g.H, tiles_n = H / 16, l = lane_id();
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     using B = RegB<K, false, 2>;
     using U = AUnits<NB, WV, 1>;
-    const uint8_t* base = expert_base(A, e);
+    const uint8_t* base = item_blob(A, a);
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base) + A.g.gu_bytes, (short)0,
                                                       (int)A.g.d_bytes, 0x00020000);
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(A.abuf, (short)0, A.npairs * 2 * I, 0x00020000);
@@ -250,11 +251,11 @@ __device__ __forceinline__ void down_rows(const GroupedArgs& A, int e, int s0, i
 
 // an item of one block: 4 waves of 64 columns (256 of H) in each of KS K-slices
 template <int K, int KS, typename TY>
-__device__ __forceinline__ void down_item(const GroupedArgs& A, int e, int s0, int rows, int nt, float* ep) {
+__device__ __forceinline__ void down_item(const GroupedArgs& A, int a, int s0, int rows, int nt, float* ep) {
     const int I = A.g.I, H = A.g.H, tiles_n = H / 16, l = lane_id();
     const int wv = uni(threadIdx.x >> 6), wc = wv & 3, ks = wv >> 2;
     using B = RegB<K, false, 2>;
-    const uint8_t* base = expert_base(A, e);
+    const uint8_t* base = item_blob(A, a);
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base) + A.g.gu_bytes, (short)0,
                                                       (int)A.g.d_bytes, 0x00020000);
     const auto ra = __builtin_amdgcn_make_buffer_rsrc(A.abuf, (short)0, A.npairs * 2 * I, 0x00020000);
@@ -289,13 +290,21 @@ __device__ __forceinline__ void down_item(const GroupedArgs& A, int e, int s0, i
 // One launch per product (two launches, one per item size, left the chip idle behind the longest item of each: a batch
 // of 64 rows took 193 us in two, 132 us in one). !BIG (items of up to 4 blocks): 4 waves per SIMD; the items of several blocks come first, then
 // those of one. BIG (items of up to 12 blocks): 2 waves per SIMD, block counts below 9 rounded up to 4, 6 or 8.
-template <int K, int WV, bool BIG>
+// FILL: the instantiations that copy (exl3_fill.cuh); the copy inside the others would cost them up to 3 % in registers.
+template <int K, int WV, bool BIG, bool FILL>
 __global__ void __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(BIG ? 2 : 4)))
 grouped_gateup_kernel(GroupedArgs A) {
     constexpr int kLds = std::max(2 * AUnits<BIG ? 12 : 4, WV, 2>::kBuf, 2 * 16 * kEpRowW<WV> * 4);
     __shared__ __align__(16) uint8_t lds[kLds];
-    const int nblk = A.g.I / (32 * WV), nmany = uni(A.n_items[BIG ? 0 : 1]);
     int blk = blockIdx.x, a, nb;
+    if constexpr (FILL) {                        // a cached call's misses: their down trellis
+        if (blk < fill_workgroups(64 * WV)) {
+            fill_part<64 * WV>(A, 1, blk);
+            return;
+        }
+        blk -= fill_workgroups(64 * WV);
+    }
+    const int nblk = A.g.I / (32 * WV), nmany = uni(A.n_items[BIG ? 0 : 1]);
     const int bmany = (nmany + 7) / 8 * 8 * nblk;
     if (BIG || blk < bmany) {
         gr_block(blk, nblk, a, nb);
@@ -305,23 +314,23 @@ grouped_gateup_kernel(GroupedArgs A) {
             gr_block(blk - bmany, A.g.I / 128, a, nb);
             a += nmany;
             if (a >= A.n_items[0]) return;
-            gateup_item<K, WV / 4>(A, uni(A.it_expert[a]), uni(A.it_start[a]), uni(A.it_cnt[a]), nb, (float*)lds);
+            gateup_item<K, WV / 4>(A, a, uni(A.it_start[a]), uni(A.it_cnt[a]), nb, (float*)lds);
         }
         return;
     }
-    const int e = uni(A.it_expert[a]), s0 = uni(A.it_start[a]), rows = uni(A.it_cnt[a]), bl = (rows + 15) >> 4;
+    const int s0 = uni(A.it_start[a]), rows = uni(A.it_cnt[a]), bl = (rows + 15) >> 4;
     if constexpr (!BIG) {
-        if (bl <= 2) gateup_rows<K, 2, WV>(A, e, s0, rows, nb, lds);
-        else if (bl == 3) gateup_rows<K, 3, WV>(A, e, s0, rows, nb, lds);
-        else gateup_rows<K, 4, WV>(A, e, s0, rows, nb, lds);
+        if (bl <= 2) gateup_rows<K, 2, WV>(A, a, s0, rows, nb, lds);
+        else if (bl == 3) gateup_rows<K, 3, WV>(A, a, s0, rows, nb, lds);
+        else gateup_rows<K, 4, WV>(A, a, s0, rows, nb, lds);
     } else {
-        if (bl <= 4) gateup_rows<K, 4, WV>(A, e, s0, rows, nb, lds);
-        else if (bl <= 6) gateup_rows<K, 6, WV>(A, e, s0, rows, nb, lds);
-        else if (bl <= 8) gateup_rows<K, 8, WV>(A, e, s0, rows, nb, lds);
-        else if (bl == 9) gateup_rows<K, 9, WV>(A, e, s0, rows, nb, lds);
-        else if (bl == 10) gateup_rows<K, 10, WV>(A, e, s0, rows, nb, lds);
-        else if (bl == 11) gateup_rows<K, 11, WV>(A, e, s0, rows, nb, lds);
-        else gateup_rows<K, 12, WV>(A, e, s0, rows, nb, lds);
+        if (bl <= 4) gateup_rows<K, 4, WV>(A, a, s0, rows, nb, lds);
+        else if (bl <= 6) gateup_rows<K, 6, WV>(A, a, s0, rows, nb, lds);
+        else if (bl <= 8) gateup_rows<K, 8, WV>(A, a, s0, rows, nb, lds);
+        else if (bl == 9) gateup_rows<K, 9, WV>(A, a, s0, rows, nb, lds);
+        else if (bl == 10) gateup_rows<K, 10, WV>(A, a, s0, rows, nb, lds);
+        else if (bl == 11) gateup_rows<K, 11, WV>(A, a, s0, rows, nb, lds);
+        else gateup_rows<K, 12, WV>(A, a, s0, rows, nb, lds);
     }
 }
 
@@ -345,24 +354,24 @@ grouped_down_kernel(GroupedArgs A) {
             gr_block(blk - bmany, A.g.H / 256, a, nt);
             a += nmany;
             if (a >= uni(A.n_items[0])) return;
-            down_item<K, WV / 4, TY>(A, uni(A.it_expert[a]), uni(A.it_start[a]), uni(A.it_cnt[a]), nt, (float*)lds);
+            down_item<K, WV / 4, TY>(A, a, uni(A.it_start[a]), uni(A.it_cnt[a]), nt, (float*)lds);
         }
         return;
     }
-    const int e = uni(A.it_expert[a]), s0 = uni(A.it_start[a]), rows = uni(A.it_cnt[a]), bl = (rows + 15) >> 4;
+    const int s0 = uni(A.it_start[a]), rows = uni(A.it_cnt[a]), bl = (rows + 15) >> 4;
     if constexpr (!BIG) {
-        if (!kOne && bl == 1) down_rows<K, 1, WV, false, TY>(A, e, s0, rows, nt, lds);
-        else if (bl <= 2) down_rows<K, 2, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else if (bl == 3) down_rows<K, 3, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else down_rows<K, 4, WV, true, TY>(A, e, s0, rows, nt, lds);
+        if (!kOne && bl == 1) down_rows<K, 1, WV, false, TY>(A, a, s0, rows, nt, lds);
+        else if (bl <= 2) down_rows<K, 2, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else if (bl == 3) down_rows<K, 3, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else down_rows<K, 4, WV, true, TY>(A, a, s0, rows, nt, lds);
     } else {
-        if (bl <= 4) down_rows<K, 4, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else if (bl <= 6) down_rows<K, 6, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else if (bl <= 8) down_rows<K, 8, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else if (bl == 9) down_rows<K, 9, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else if (bl == 10) down_rows<K, 10, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else if (bl == 11) down_rows<K, 11, WV, true, TY>(A, e, s0, rows, nt, lds);
-        else down_rows<K, 12, WV, true, TY>(A, e, s0, rows, nt, lds);
+        if (bl <= 4) down_rows<K, 4, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else if (bl <= 6) down_rows<K, 6, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else if (bl <= 8) down_rows<K, 8, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else if (bl == 9) down_rows<K, 9, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else if (bl == 10) down_rows<K, 10, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else if (bl == 11) down_rows<K, 11, WV, true, TY>(A, a, s0, rows, nt, lds);
+        else down_rows<K, 12, WV, true, TY>(A, a, s0, rows, nt, lds);
     }
 }
 
@@ -371,21 +380,26 @@ void launch_products(const GroupedArgs& a, bool y32, hipStream_t s) {
     const size_t np = a.npairs, mi = grouped_max_items(np, a.E);
     auto g8 = [](size_t items) { return (unsigned)((items + 7) / 8 * 8); };
     const int I = a.g.I, H = a.g.H;
-    const bool big = a.rmax > 64;                // (8-wave layouts and fp16 outputs only: grouped_rmax)
+    const bool big = a.rmax > 64;                // (8-wave layouts and fp16 outputs only, moe_grouped.hip)
     auto run = [&](auto kern, unsigned grid, int nt) { hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), 0, s, a); };
     // items of several blocks hold at least 17 rows each
-    const unsigned many = g8(np / 17);
-    if (I % 256 == 0) {
-        if (big) run(grouped_gateup_kernel<K, 8, true>, g8(mi) * (I / 256), 512);
-        else run(grouped_gateup_kernel<K, 8, false>, many * (I / 256) + g8(std::min<size_t>(np, a.E)) * (I / 128), 512);
+    const unsigned many = g8(np / 17), one = g8(std::min<size_t>(np, a.E));
+    if (big) {
+        run(grouped_gateup_kernel<K, 8, true, false>, g8(mi) * (I / 256), 512);
+    } else if (I % 256 == 0) {
+        const unsigned grid = many * (I / 256) + one * (I / 128);
+        if (a.f.list) run(grouped_gateup_kernel<K, 8, false, true>, fill_workgroups(512) + grid, 512);
+        else run(grouped_gateup_kernel<K, 8, false, false>, grid, 512);
     } else {
-        run(grouped_gateup_kernel<K, 4, false>, (many + g8(std::min<size_t>(np, a.E))) * (I / 128), 256);
+        const unsigned grid = (many + one) * (I / 128);
+        if (a.f.list) run(grouped_gateup_kernel<K, 4, false, true>, fill_workgroups(256) + grid, 256);
+        else run(grouped_gateup_kernel<K, 4, false, false>, grid, 256);
     }
     auto down = [&](auto ty) {
         using TY = decltype(ty);
-        const unsigned one = g8(std::min<size_t>(np, a.E)) * (H / 256);
-        if (H % 512 == 0) run(grouped_down_kernel<K, 8, false, TY>, y32 ? many * (H / 512) + one : g8(mi) * (H / 512), 512);
-        else run(grouped_down_kernel<K, 4, false, TY>, y32 ? many * (H / 256) + one : g8(mi) * (H / 256), 256);
+        const unsigned ones = one * (H / 256);
+        if (H % 512 == 0) run(grouped_down_kernel<K, 8, false, TY>, y32 ? many * (H / 512) + ones : g8(mi) * (H / 512), 512);
+        else run(grouped_down_kernel<K, 4, false, TY>, y32 ? many * (H / 256) + ones : g8(mi) * (H / 256), 256);
     };
     if (big) run(grouped_down_kernel<K, 8, true, half_t>, g8(mi) * (H / 512), 512);
     else if (y32) down(float{});

@@ -104,3 +104,32 @@ def test_static_entry_matches_cached(fused):
         torch.cuda.synchronize()
     finally:
         lib.exl3_set_fused_ensure(1)
+
+
+def test_static_entry_of_the_grouped_sizes():
+    """12 and 25 rows (the largest call that the static array admits), where both entries run the grouped kernels, among
+    smaller calls that do not: outputs, routing and cache state are those of the cached entry, and the grouped calls' own
+    scratch leaves the exchange words of the small ones alone. 25 rows pick more experts than there are slots."""
+    from exl3xpu import capi
+    lib = capi.lib()
+    print("case no-alloc entry, grouped sizes", flush=True)
+    stores = _stores()
+    stores[0]._bind_strides()
+    for rc in (lib.exl3_set_tier(None, None, 0, None), lib.exl3_set_victims(None),
+               lib.exl3_set_prefetch_commit(None, None, 0), lib.exl3_set_decision_log(None, 0)):
+        assert rc == 0
+    assert 12 * TOPK * I >= 56000
+    for n, M in enumerate((12, 2, 25, 1, 12, 25, 4)):
+        x, ids, w = _inputs(M, 300 + n)
+        got = []
+        for s, st in enumerate(stores):
+            out, it, wt = torch.full_like(x, float("nan")), ids.clone(), w.clone()
+            ws = torch.empty(lib.exl3_moe_forward_workspace(M, H, I, TOPK, E), dtype=torch.uint8, device="cuda")
+            rc = _call(lib, st, n % 2, x, it, wt, out, static=(s == 1), ws=ws)
+            assert rc == 0, lib.exl3_last_error().decode()
+            got.append((out, it, wt))
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(*got)), (n, M)
+        for t in ("slot_of_dev", "slot_key", "slot_last", "tick", "fill_list", "fill_all"):
+            assert torch.equal(getattr(stores[0], t), getattr(stores[1], t)), (n, M, t)
+        assert not stores[0].fill_all.any()
