@@ -119,6 +119,13 @@ size_t exl3_moe_forward_workspace(int M, int H, int I, int topk, int n_experts);
 int exl3_moe_forward(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
                      const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
                      int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream);
+/* The same call for a table some of whose experts are in host memory (the same results, bit for bit, and the same
+ * workspace): blobs outside the device memory [hbm_base, hbm_base + hbm_bytes) may be. At the prefill sizes the kernels
+ * then read each of those over PCIe as few times as they can. */
+int exl3_moe_forward_host(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
+                          const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
+                          int64_t out_stride, void* workspace, size_t workspace_bytes, int64_t hbm_base,
+                          int64_t hbm_bytes, void* stream);
 
 /* moe_forward_cached (a8:1229-1261): the same through the device-managed expert cache of layer `layer`:
  * ensure (tier mask, hits, exact-LRU victims, assignment) -> victim write-back -> GEMVs with write-through of misses

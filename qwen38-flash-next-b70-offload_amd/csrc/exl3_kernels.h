@@ -111,6 +111,10 @@ struct GroupedArgs {
     int64_t* it_blob; int* it_start; int* it_cnt;  // items: up to rmax sorted positions of one expert (its blob), longest
                                                    // first
     int* n_items;                                  // [2] items, and those of more than 16 rows (the first ones)
+    // blobs outside [hbm_lo, hbm_hi) may be in host memory (hbm_hi 0: nothing is known of the table); items of those of more
+    // than 64 rows apart, up to 192 rows each (big_n null: none)
+    int64_t hbm_lo, hbm_hi;
+    int64_t* big_blob; int* big_start; int* big_cnt; int* big_n;
     _Float16* suh;                                 // [E][2][H] input scales of the experts in use, or null: in the blobs
     _Float16* xh;                                  // [npairs][2][H] input Hadamards (gate, up)
     _Float16* abuf;                                // [npairs][I]

@@ -342,7 +342,7 @@ static int forward_impl(const void* x, int x_dtype, int64_t x_stride, int M, int
                         size_t ws_bytes, hipStream_t st, const int64_t* fill, int64_t* commit_ptrs, int64_t* commit_fill,
                         const int32_t* fill_list, const int64_t* pair_ptr, const VictimArgs* va = nullptr,
                         int max_victims = 0, const EnsureArgs* fused_ens = nullptr, bool vict_inline = false,
-                        uint64_t* xb_given = nullptr, const FillArgs* fills = nullptr) {
+                        uint64_t* xb_given = nullptr, const FillArgs* fills = nullptr, const int64_t* hbm = nullptr) {
     if (!fill && use_prefill(M, topk)) {
         if (H % 256) return fail(EXL3_EUNSUPPORTED, "moe prefill: H %% 256 == 0 required (H=%d)", H);
         if ((int64_t)M * topk > (1 << 28)) return fail(EXL3_EUNSUPPORTED, "moe prefill: %d x %d pairs", M, topk);
@@ -366,6 +366,10 @@ static int forward_impl(const void* x, int x_dtype, int64_t x_stride, int M, int
         ga.out_stride = out_stride;
         ga.g = blob_geom(H, I, K);
         if (fills) ga.f = *fills;
+        if (hbm) {
+            ga.hbm_lo = hbm[0];
+            ga.hbm_hi = hbm[1];
+        }
         const hipError_t e = launch_grouped(ga, y32, ws, st);
         return e == hipSuccess ? EXL3_OK : hip_fail(e, "moe grouped launch");
     }
@@ -421,9 +425,9 @@ static int forward_impl(const void* x, int x_dtype, int64_t x_stride, int M, int
     return EXL3_OK;
 }
 
-int exl3_moe_forward(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
-                     const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
-                     int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream) {
+static int forward_checked(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
+                           const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
+                           int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream, const int64_t* hbm) {
     if (M < 0 || topk <= 0) return fail(EXL3_EINVAL, "moe_forward: M=%d topk=%d", M, topk);
     if (x_dtype < EXL3_DT_F16 || x_dtype > EXL3_DT_F32) return fail(EXL3_EINVAL, "moe_forward: x dtype");
     int r = check_geometry(H, I, K, n_experts);
@@ -431,7 +435,25 @@ int exl3_moe_forward(const void* x, int x_dtype, int64_t x_stride, int M, int H,
     if (M == 0) return EXL3_OK;
     if (!x || !topk_ids || !topk_w || !ptrs || !out) return fail(EXL3_EINVAL, "moe_forward: null pointer");
     return forward_impl(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs, I, K, n_experts, out, out_stride,
-                        workspace, workspace_bytes, (hipStream_t)stream, nullptr, nullptr, nullptr, nullptr, nullptr);
+                        workspace, workspace_bytes, (hipStream_t)stream, nullptr, nullptr, nullptr, nullptr, nullptr,
+                        nullptr, 0, nullptr, false, nullptr, nullptr, hbm);
+}
+
+int exl3_moe_forward(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
+                     const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
+                     int64_t out_stride, void* workspace, size_t workspace_bytes, void* stream) {
+    return forward_checked(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs, I, K, n_experts, out, out_stride,
+                           workspace, workspace_bytes, stream, nullptr);
+}
+
+int exl3_moe_forward_host(const void* x, int x_dtype, int64_t x_stride, int M, int H, const int32_t* topk_ids,
+                          const float* topk_w, int topk, const int64_t* ptrs, int I, int K, int n_experts, void* out,
+                          int64_t out_stride, void* workspace, size_t workspace_bytes, int64_t hbm_base,
+                          int64_t hbm_bytes, void* stream) {
+    if (hbm_bytes < 0) return fail(EXL3_EINVAL, "moe_forward_host: hbm_bytes=%lld", (long long)hbm_bytes);
+    const int64_t hbm[2] = {hbm_base, std::max<int64_t>(hbm_base + hbm_bytes, 1)};
+    return forward_checked(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs, I, K, n_experts, out, out_stride,
+                           workspace, workspace_bytes, stream, hbm);
 }
 
 int exl3_moe_prefetch(const int32_t* ids, int n_ids, int64_t* ptrs_all, int layer, int32_t* slot_of,
@@ -612,8 +634,9 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
     if (M >= g_cfg.prefill_min_m || n_slots == 0) {
         if (xb) return fail(EXL3_EUNSUPPORTED, "moe_forward_cached_static: M=%d n_slots=%d takes the uncached path, "
                             "which needs a workspace (use exl3_moe_forward_cached)", M, n_slots);
-        return exl3_moe_forward(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs_all + (int64_t)layer * E, I, K,
-                                E, out, out_stride, workspace, workspace_bytes, stream);
+        return exl3_moe_forward_host(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs_all + (int64_t)layer * E,
+                                     I, K, E, out, out_stride, workspace, workspace_bytes, slot_base,
+                                     n_slots * (g_cfg.slot_stride ? g_cfg.slot_stride : blob_geom(H, I, K).blob), stream);
     }
     if (!slot_of || !slot_key || !slot_last || !tick || !host_base || !fill_all || !fill_list)
         return fail(EXL3_EINVAL, "moe_forward_cached: null cache state");
@@ -698,9 +721,10 @@ static int cached_impl(const void* x, int x_dtype, int64_t x_stride, int M, int 
             f.sstride = ea.blob;
             f.ram_res = vict_res;
         }
+        const int64_t hbm[2] = {slot_base, slot_base + n_slots * ea.blob};
         return forward_impl(x, x_dtype, x_stride, M, H, topk_ids, topk_w, topk, ptrs_all + (int64_t)layer * E, I, K, E,
                             out, out_stride, workspace, workspace_bytes, st, nullptr, nullptr, nullptr, nullptr, nullptr,
-                            nullptr, 0, nullptr, false, nullptr, &f);
+                            nullptr, 0, nullptr, false, nullptr, &f, hbm);
     }
     const size_t need = decode_workspace_bytes(P, H, I);
     if (!workspace || workspace_bytes < need)

@@ -64,16 +64,23 @@ __device__ __forceinline__ uint64_t block_scan64(uint64_t v, uint64_t* sw, uint6
 
 // thread e: the items of expert e (tot rows from sorted position st): the fewest items of at most rmax rows, cut evenly
 // in 16-row blocks; ordered by descending block count over all experts (packed scans of 16 bits per block count), so
-// that the longest start first. n_items[0]: all items, [1]: those of more than one block.
+// that the longest start first. n_items[0]: all items, [1]: those of more than one block. With big_n, the experts outside
+// [hbm_lo, hbm_hi) of more than 64 rows are cut at 192 rows (5 blocks and more) into a list of their own.
 __device__ __forceinline__ void emit_items(const GroupedArgs& A, int e, int st, int tot, uint64_t* sw) {
-    const int n = (tot + A.rmax - 1) / A.rmax, nb = n ? ((tot + n - 1) / n + 15) >> 4 : 0;   // items, blocks of each
-    int above = 0;
     int64_t blob = 0;
-    if (n) {                                     // (a miss of a cached call: its new slot)
+    if (tot) {                                   // (a miss of a cached call: its new slot)
         blob = A.ptrs[e];
         if (A.f.list && A.f.fill[e]) blob = A.f.fill[e];
     }
-    for (int g = (A.rmax + 63) / 64 - 1; g >= 0; --g) {          // block counts 4 g + 1 .. 4 g + 4
+    const int rmax = A.big_n && tot > 64 && (blob < A.hbm_lo || blob >= A.hbm_hi) ? 192 : A.rmax;
+    const int n = (tot + rmax - 1) / rmax, nb = n ? ((tot + n - 1) / n + 15) >> 4 : 0;       // items, blocks of each
+    int above = 0;
+    for (int g = A.big_n ? 2 : (A.rmax + 63) / 64 - 1; g >= 0; --g) {      // block counts 4 g + 1 .. 4 g + 4
+        const bool big = A.big_n && g > 0;
+        if (A.big_n && g == 0) {
+            if (threadIdx.x == 0) A.big_n[0] = above;
+            above = 0;
+        }
         uint64_t tt;
         const uint64_t ex = block_scan64(nb > 4 * g && nb <= 4 * g + 4 ? (uint64_t)n << (16 * (nb - 1 - 4 * g)) : 0ull, sw, tt);
 #pragma unroll
@@ -81,9 +88,9 @@ __device__ __forceinline__ void emit_items(const GroupedArgs& A, int e, int st, 
             if (4 * g + k == nb) {
                 int p = above + (int)((ex >> (16 * (k - 1))) & 0xFFFF);
                 for (int i = 0; i < n; ++i, ++p) {
-                    A.it_blob[p] = blob;
-                    A.it_start[p] = st + i * 16 * nb;
-                    A.it_cnt[p] = min(16 * nb, tot - i * 16 * nb);
+                    (big ? A.big_blob : A.it_blob)[p] = blob;
+                    (big ? A.big_start : A.it_start)[p] = st + i * 16 * nb;
+                    (big ? A.big_cnt : A.it_cnt)[p] = min(16 * nb, tot - i * 16 * nb);
                 }
             }
             if (g == 0 && k == 1 && threadIdx.x == 0) A.n_items[1] = above;
@@ -289,14 +296,19 @@ static int pass_rows(int M, int topk, int H, int I) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(M, np / topk));
 }
 
-// (up to 16 picks per expert the scales are at most 5 % of what an expert's products read; the workspace has room for
-// min(E, np / 16) experts' scales, which grows with both)
-static bool grouped_scales(size_t np, int E) { return np > (size_t)16 * E; }
+// The scales are copied from 2 picks per expert on where experts may be in host memory (300 tokens, a third of the experts
+// there: 3,805 us without, 3,755 with the copies), else from 16 on, for a table of unknown make (301 tokens in HBM: 235
+// without, 240 us with them). The workspace has room for min(E, np / 2) experts' scales (np / 16 at the decode sizes, which
+// copy from 16 on), which grows with both
+static bool grouped_scales(size_t np, int E, bool host) { return np > (size_t)(host ? 2 : 16) * E; }
+// the lists of an upper bound of n items and their counts
+static size_t list_bytes(size_t n) { return align256((4 * n + 2) * 4); }
+static size_t big_items(size_t np) { return np / 65; }           // (an expert of more than 64 rows has 65 or more per item)
 
 size_t grouped_workspace_bytes(int M, int topk, int H, int I, int E, bool y32) {
     const size_t np = (size_t)pass_rows(M, topk, H, I) * topk;
-    return align256((4 * grouped_max_items(np, E) + 2) * 4) + align256(np * 4) + align256(np * 4 * H) + align256(np * 2 * I) +
-           align256(np * H * (y32 ? 4 : 2)) + align256(std::min<size_t>(E, np / 16) * 4 * H);
+    return list_bytes(grouped_max_items(np, E)) + (y32 ? 0 : list_bytes(big_items(np))) + align256(np * 4) + align256(np * 4 * H) + align256(np * 2 * I) +
+           align256(np * H * (y32 ? 4 : 2)) + align256(std::min<size_t>(E, np / (y32 ? 16 : 2)) * 4 * H);
 }
 
 static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) {
@@ -304,20 +316,34 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
     // Items of up to 64 rows run 4 waves per SIMD; of up to 192 rows 2 (the accumulators), but decode once where the
     // others decode three times. With 56 rows per expert on average and more, 64-row items would cut most experts
     // (H 4096 / I 1536 / K 2, 777 tokens of 49 rows per expert: 64-row items 533 us, items of up to 128 rows 603 us).
-    a.rmax = np > (size_t)56 * a.E && a.g.I % 256 == 0 && a.g.H % 512 == 0 && !y32 ? 192 : 64;
+    const bool host = a.hbm_hi != 0 && !y32, large = a.g.I % 256 == 0 && a.g.H % 512 == 0 && !y32;
+    a.rmax = large && np > (size_t)56 * a.E ? 192 : 64;
     uint8_t* p = (uint8_t*)ws;
     auto take = [&p](size_t n) { uint8_t* q = p; p += align256(n); return q; };
-    int* it = (int*)take((4 * mi + 2) * 4);
+    int* it = (int*)take(list_bytes(mi));
     a.it_blob = (int64_t*)it;
     a.it_start = it + 2 * mi;
     a.it_cnt = it + 3 * mi;
     a.n_items = it + 4 * mi;
+    // Experts in host memory: each 64-row item would read its expert over PCIe again, so those of more rows run as items of
+    // up to 192 rows in launches of their own; only those, since the reads of the others would wait for the HBM experts'
+    // items among them. H 2048 / I 512 / K 3, Zipf tokens, a third of the experts in host memory, us without and with: 700
+    // tokens 4,104 and 3,780, 1,500 4,592 and 4,013, 2,600 4,857 and 4,190; H 4096 / I 1536 / K 4, 777 tokens 9,835 and 7,750.
+    // With every expert in HBM the added launches and the copied scales cost 3-10 us (301 tokens 235 and 243).
+    if (host && large && a.rmax == 64) {
+        const size_t mb = big_items(np);
+        int* b = (int*)take(list_bytes(mb));
+        a.big_blob = (int64_t*)b;
+        a.big_start = b + 2 * mb;
+        a.big_cnt = b + 3 * mb;
+        a.big_n = b + 4 * mb;
+    }
     a.perm = (int*)take(np * 4);
     a.xh = (half_t*)take(np * 4 * a.g.H);
     a.abuf = (half_t*)take(np * 2 * a.g.I);
     a.y = take(np * a.g.H * (y32 ? 4 : 2));
     a.suh = nullptr;
-    if (grouped_scales(np, a.E)) {
+    if (grouped_scales(np, a.E, host)) {
         a.suh = (half_t*)take((size_t)a.E * 4 * a.g.H);
         hipLaunchKernelGGL(grouped_scales_kernel, dim3((unsigned)((a.E + kScaleExperts - 1) / kScaleExperts)), dim3(1024), 0, s, a);
     }

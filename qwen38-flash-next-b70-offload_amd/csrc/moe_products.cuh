@@ -382,6 +382,15 @@ void launch_products(const GroupedArgs& a, bool y32, hipStream_t s) {
     const int I = a.g.I, H = a.g.H;
     const bool big = a.rmax > 64;                // (8-wave layouts and fp16 outputs only, moe_grouped.hip)
     auto run = [&](auto kern, unsigned grid, int nt) { hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), 0, s, a); };
+    GroupedArgs b = a;                           // the experts of more than 64 rows, where they are listed apart
+    b.it_blob = a.big_blob;
+    b.it_start = a.big_start;
+    b.it_cnt = a.big_cnt;
+    b.n_items = a.big_n;
+    auto apart = [&](auto kern, int blocks) {
+        if (a.big_n && np > 64) hipLaunchKernelGGL(kern, dim3(g8(np / 65) * blocks), dim3(512), 0, s, b);
+    };
+    apart(grouped_gateup_kernel<K, 8, true, false>, I / 256);
     // items of several blocks hold at least 17 rows each
     const unsigned many = g8(np / 17), one = g8(std::min<size_t>(np, a.E));
     if (big) {
@@ -395,6 +404,7 @@ void launch_products(const GroupedArgs& a, bool y32, hipStream_t s) {
         if (a.f.list) run(grouped_gateup_kernel<K, 4, false, true>, fill_workgroups(256) + grid, 256);
         else run(grouped_gateup_kernel<K, 4, false, false>, grid, 256);
     }
+    apart(grouped_down_kernel<K, 8, true, half_t>, H / 512);
     auto down = [&](auto ty) {
         using TY = decltype(ty);
         const unsigned ones = one * (H / 256);

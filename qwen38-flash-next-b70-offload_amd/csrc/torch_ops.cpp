@@ -30,8 +30,8 @@ int dtype_code(const at::Tensor& x) {
     TORCH_CHECK(false, "x dtype: bf16, fp16 or fp32 expected, got ", x.scalar_type());
 }
 
-at::Tensor moe_forward(at::Tensor x, at::Tensor topk_ids, at::Tensor topk_w, at::Tensor ptrs, int64_t I, int64_t K,
-                       int64_t n_experts) {
+at::Tensor forward_checked(const at::Tensor& x, const at::Tensor& topk_ids, const at::Tensor& topk_w,
+                           const at::Tensor& ptrs, int64_t I, int64_t K, int64_t n_experts, const int64_t* hbm) {
     TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "moe_forward: x must be [M, H] with unit column stride");
     TORCH_CHECK(topk_ids.scalar_type() == at::kInt && topk_ids.is_contiguous(), "moe_forward: topk_ids int32 contiguous");
     TORCH_CHECK(topk_w.scalar_type() == at::kFloat && topk_w.is_contiguous(), "moe_forward: topk_w fp32 contiguous");
@@ -43,11 +43,27 @@ at::Tensor moe_forward(at::Tensor x, at::Tensor topk_ids, at::Tensor topk_w, at:
     if (M == 0) return out;
     const size_t ws = exl3_moe_forward_workspace(M, H, (int)I, topk, (int)n_experts);
     auto w = at::empty({(int64_t)ws}, x.options().dtype(at::kByte));
-    check(exl3_moe_forward(x.data_ptr(), dtype_code(x), x.stride(0), M, H, topk_ids.data_ptr<int>(),
-                           topk_w.data_ptr<float>(), topk, ptrs.data_ptr<int64_t>(), (int)I, (int)K, (int)n_experts,
-                           out.data_ptr(), out.stride(0), w.data_ptr(), ws, cur_stream(x)),
+    const int32_t* ids = topk_ids.data_ptr<int>();
+    const int64_t* table = ptrs.data_ptr<int64_t>();
+    check(hbm ? exl3_moe_forward_host(x.data_ptr(), dtype_code(x), x.stride(0), M, H, ids, topk_w.data_ptr<float>(), topk,
+                                      table, (int)I, (int)K, (int)n_experts, out.data_ptr(), out.stride(0), w.data_ptr(),
+                                      ws, hbm[0], hbm[1], cur_stream(x))
+              : exl3_moe_forward(x.data_ptr(), dtype_code(x), x.stride(0), M, H, ids, topk_w.data_ptr<float>(), topk,
+                                 table, (int)I, (int)K, (int)n_experts, out.data_ptr(), out.stride(0), w.data_ptr(), ws,
+                                 cur_stream(x)),
           "moe_forward");
     return out;
+}
+
+at::Tensor moe_forward(at::Tensor x, at::Tensor topk_ids, at::Tensor topk_w, at::Tensor ptrs, int64_t I, int64_t K,
+                       int64_t n_experts) {
+    return forward_checked(x, topk_ids, topk_w, ptrs, I, K, n_experts, nullptr);
+}
+// the same for a table with experts in host memory (outside the device memory [hbm_base, hbm_base + hbm_bytes))
+at::Tensor moe_forward_host(at::Tensor x, at::Tensor topk_ids, at::Tensor topk_w, at::Tensor ptrs, int64_t I, int64_t K,
+                            int64_t n_experts, int64_t hbm_base, int64_t hbm_bytes) {
+    const int64_t hbm[2] = {hbm_base, hbm_bytes};
+    return forward_checked(x, topk_ids, topk_w, ptrs, I, K, n_experts, hbm);
 }
 
 // moe_prefetch (a8:1194-1222): claim slots for predicted experts of `layer`, copy them from host, repoint the table,
@@ -462,6 +478,9 @@ TORCH_LIBRARY(exl3xpu_C, m) {
 TORCH_LIBRARY(exl3xpu_moe, m) {
     m.def("moe_forward(Tensor x, Tensor topk_ids, Tensor topk_w, Tensor ptrs, int I, int K, int n_experts) -> Tensor");
     m.impl("moe_forward", c10::DispatchKey::CUDA, &moe_forward);
+    m.def("moe_forward_host(Tensor x, Tensor topk_ids, Tensor topk_w, Tensor ptrs, int I, int K, int n_experts, "
+          "int hbm_base, int hbm_bytes) -> Tensor");
+    m.impl("moe_forward_host", c10::DispatchKey::CUDA, &moe_forward_host);
     m.def("moe_forward_cached(Tensor x, Tensor(i!) topk_ids, Tensor(j!) topk_w, Tensor(a!) ptrs_all, int layer, "
           "Tensor(b!) slot_of, Tensor(c!) slot_key, Tensor(d!) slot_last, Tensor(e!) tick, Tensor host_base, "
           "int slot_base, Tensor(f!) fill_all, Tensor(g!) fill_list, int max_fill, int I, int K, int n_experts, "

@@ -37,6 +37,8 @@ SIGNATURES = {
     "exl3_moe_forward_workspace": (c_sz, [c_i32, c_i32, c_i32, c_i32, c_i32]),
     "exl3_moe_forward": (c_i32, [c_p, c_i32, c_i64, c_i32, c_i32, c_p, c_p, c_i32, c_p, c_i32, c_i32, c_i32, c_p, c_i64,
                                  c_p, c_sz, c_p]),
+    "exl3_moe_forward_host": (c_i32, [c_p, c_i32, c_i64, c_i32, c_i32, c_p, c_p, c_i32, c_p, c_i32, c_i32, c_i32, c_p,
+                                      c_i64, c_p, c_sz, c_i64, c_i64, c_p]),
     "exl3_moe_forward_cached": (c_i32, [c_p, c_i32, c_i64, c_i32, c_i32, c_p, c_p, c_i32, c_p, c_i32, c_p, c_p, c_p, c_p,
                                         c_i32, c_p, c_i64, c_p, c_p, c_i32, c_i32, c_i32, c_i32, c_p, c_i64, c_p, c_sz,
                                         c_p]),

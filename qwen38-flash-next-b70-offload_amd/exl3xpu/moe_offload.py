@@ -44,7 +44,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _ops_lock = threading.Lock()
 _ops_ns = None
 # ops whose meta output is shaped like x (registered for torch.compile / fake tensors)
-_X_SHAPED_OPS = ("moe_forward", "moe_forward_cached")
+_X_SHAPED_OPS = ("moe_forward", "moe_forward_host", "moe_forward_cached")
 
 # Staged prefill (copy-stream streaming into HBM staging buffers) has been verified on the GPU with staging buffers of
 # up to this many bytes per layer. A full-size run (8,192 tokens x 48 layers, 512 experts of 1.2 MB) ended in a GPU
@@ -644,7 +644,10 @@ class ExpertStore:
     def forward(self, key, x: torch.Tensor, topk_ids: torch.Tensor, topk_w: torch.Tensor, ptrs=None) -> torch.Tensor:
         self._watch.check("exl3xpu.forward")
         ids, w = self._routing(topk_ids, topk_w)
-        return self.X.moe_forward(x, ids, w, self.ptrs(key) if ptrs is None else ptrs, self.I, self.k_of(key), self.E)
+        args = (x, ids, w, self.ptrs(key) if ptrs is None else ptrs, self.I, self.k_of(key), self.E)
+        if self.n_slots >= len(self.layer_index) * self.E:
+            return self.X.moe_forward(*args)
+        return self.X.moe_forward_host(*args, self.slot_base, self.n_slots * self.slot_stride)   # host records among them
 
     def forward_cached(self, key, x: torch.Tensor, topk_ids: torch.Tensor, topk_w: torch.Tensor,
                        max_fill: int | None = None) -> torch.Tensor:

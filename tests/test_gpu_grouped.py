@@ -119,3 +119,34 @@ def test_grouped_scales_only_of_the_experts_in_use():
     finally:
         _ops().moe_set_prefill_min_m(256)
     assert torch.equal(a, b) and torch.equal(a, c)
+
+
+@pytest.mark.parametrize("H,I,K,where", [(512, 256, 3, "host"), (512, 256, 3, "mixed"), (1024, 512, 2, "mixed"),
+                                         (512, 256, 4, "hbm"), (768, 256, 3, "mixed"), (512, 384, 2, "mixed")])
+def test_grouped_host_experts(H, I, K, where):
+    """moe_forward_host (experts in pinned host memory: more rows per item, the input scales copied from 2 picks per expert
+    on) gives the bits of moe_forward on HBM copies, at the edges of its cuts (64 and 192 rows), also at the widths whose
+    items stay at 64 rows and where every expert counts as a host one; experts without picks have no blob."""
+    counts = [1, 16, 17, 64, 65, 80, 81, 97, 129, 176, 177, 192, 193, 385, 400, 0, 2, 33, 48, 1] + [3, 0, 5, 1] * 8
+    E, seed = len(counts), 9500 + H + I + K
+    print(f"case grouped host experts H={H} I={I} K={K} {where} E={E}", flush=True)
+    ids = _ids_of(counts, seed)
+    M = ids.shape[0]
+    assert 2 * E < M <= 56 * E
+    blobs = np.stack([synth.expert_blob(seed, e, H, I, K) for e in range(E)])
+    dev, host = torch.from_numpy(blobs).cuda(), torch.from_numpy(blobs).pin_memory()
+    full = torch.tensor([dev[e].data_ptr() for e in range(E)], dtype=torch.int64)
+    in_host = {"host": lambda e: True, "mixed": lambda e: e % 2 == 0, "hbm": lambda e: False}[where]
+    some = torch.tensor([0 if not counts[e] else (host if in_host(e) else dev)[e].data_ptr() for e in range(E)],
+                        dtype=torch.int64)
+    x = torch.from_numpy(exl3.bf16_to_f32(synth.activations(seed, M, H))).cuda().to(torch.bfloat16)
+    it = torch.from_numpy(ids).cuda()
+    wt = torch.rand(M, 1, generator=torch.Generator().manual_seed(1)).cuda()
+    _ops().moe_set_prefill_min_m(1)
+    try:
+        a = _ops().moe_forward(x, it, wt, full.cuda(), I, K, E)
+        b, c = (_ops().moe_forward_host(x, it, wt, some.cuda(), I, K, E, *hbm) for hbm in ((dev.data_ptr(), dev.numel()), (0, 0)))
+        torch.cuda.synchronize()
+    finally:
+        _ops().moe_set_prefill_min_m(256)
+    assert torch.isfinite(a.float()).all() and torch.equal(a, b) and torch.equal(a, c)
