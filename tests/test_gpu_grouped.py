@@ -1,7 +1,7 @@
 """GPU parity of the grouped expert kernels (csrc/moe_grouped.hip) where they can go wrong: rows per expert at the edges
 of the 16-row blocks and of the item cuts (64 and 192 rows), widths that take the 4- and the 8-wave workgroups, every
-bitrate, activations at odd addresses, fp32 and fp16 pick outputs, ids outside the table; against the oracle's rounding
-points within the repository's rel-L2 2e-3 (bf16 and fp16 rounding of the outputs alone are 1.7e-3 and 0.2e-3)."""
+bitrate, activations at odd addresses, fp32 and fp16 pick outputs, ids outside the table, experts in host memory, calls of
+several passes; against the oracle's rounding points within the repository's rel-L2 2e-3 (bf16 and fp16 rounding of the outputs alone are 1.7e-3 and 0.2e-3)."""
 import numpy as np
 import pytest
 import torch
@@ -150,3 +150,60 @@ def test_grouped_host_experts(H, I, K, where):
     finally:
         _ops().moe_set_prefill_min_m(256)
     assert torch.isfinite(a.float()).all() and torch.equal(a, b) and torch.equal(a, c)
+
+
+# decode sizes: up to 1,024 picks and 256 rows; one-block items beside items of 2, 3 and 4 blocks, and cut experts
+CUT_DECODE = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 97, 129, 0, 2, 3, 5, 8, 40, 22, 21]
+
+
+@pytest.mark.parametrize("H,I,K", [(512, 256, 3), (256, 128, 3), (768, 256, 2), (512, 384, 4), (1024, 512, 4)])
+def test_grouped_decode_sizes_of_every_block_count(H, I, K):
+    """Decode sizes (fp32 pick outputs, two K-slices for the items of one block) with experts of 1 to 129 rows, 4 picks a row;
+    widths that take the 4-wave and the 8-wave workgroups of both products; against the oracle's decode variant."""
+    E, seed = len(CUT_DECODE), 9600 + H + I + K
+    n = sum(CUT_DECODE)
+    assert n % 4 == 0 and n <= 1024 and n // 4 <= 256 and n * I >= 56000
+    print(f"case grouped decode block counts H={H} I={I} K={K} picks={n}", flush=True)
+    ids = _ids_of(CUT_DECODE, seed).reshape(-1, 4)
+    M = ids.shape[0]
+    w = np.random.default_rng(seed + 1).uniform(0.1, 1.0, size=(M, 4)).astype(np.float32)
+    blobs = np.stack([synth.expert_blob(seed, e, H, I, K) for e in range(E)])
+    ews = {e: exl3.ExpertWeights(blobs[e], H, I, K) for e in range(E)}
+    dev = torch.from_numpy(blobs).cuda()
+    table = torch.tensor([dev[e].data_ptr() for e in range(E)], dtype=torch.int64, device="cuda")
+    x = synth.activations(seed, M, H)
+    _, of = exl3.moe_forward(x, ids, w, ews, variant="decode")
+    xf = torch.from_numpy(exl3.bf16_to_f32(x)).cuda()
+    it, wt = torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda()
+    got, again = (_ops().moe_forward(xf, it, wt, table, I, K, E) for _ in range(2))
+    torch.cuda.synchronize()
+    assert torch.equal(got, again)
+    got = got.cpu().numpy()
+    err = np.linalg.norm((got - of).astype(np.float64), axis=1) / np.linalg.norm(of.astype(np.float64), axis=1)
+    print(f"grouped decode block counts: rel-L2 {_rel(got, of):.2e}, worst row {err.max():.2e}")
+    assert np.isfinite(got).all() and _rel(got, of) <= TOL and err.max() <= 2 * TOL
+
+
+def test_grouped_rows_of_several_passes():
+    """More picks than one pass takes (65,535 at H 8192): 4,200 rows x 16 picks run as 4,095 rows and 105 in one workspace;
+    rows on both sides of the boundary against the oracle."""
+    H, I, K, E, M, TK, seed = 8192, 128, 2, 20, 4200, 16, 9700
+    print("case grouped several passes", flush=True)
+    rng = np.random.default_rng(seed)
+    ids = np.argsort(rng.random((M, E)), axis=1)[:, :TK].astype(np.int32)
+    w = rng.uniform(0.1, 1.0, size=(M, TK)).astype(np.float32)
+    blobs = np.stack([synth.expert_blob(seed, e, H, I, K) for e in range(E)])
+    dev = torch.from_numpy(blobs).cuda()
+    table = torch.tensor([dev[e].data_ptr() for e in range(E)], dtype=torch.int64, device="cuda")
+    x = synth.activations(seed, M, H)
+    out = _ops().moe_forward(torch.from_numpy(exl3.bf16_to_f32(x)).cuda(), torch.from_numpy(ids).cuda(),
+                             torch.from_numpy(w).cuda(), table, I, K, E)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.isfinite(got).all()
+    rows = np.array([0, 4093, 4094, 4095, 4096, 4199])
+    ews = {e: exl3.ExpertWeights(blobs[e], H, I, K) for e in range(E)}
+    _, of = exl3.moe_forward(x[rows], ids[rows], w[rows], ews, variant="prefill")
+    err = np.linalg.norm((got[rows] - of).astype(np.float64), axis=1) / np.linalg.norm(of.astype(np.float64), axis=1)
+    print(f"grouped several passes: rows {rows.tolist()} rel-L2 {np.array2string(err, precision=2)}")
+    assert err.max() <= 2 * TOL

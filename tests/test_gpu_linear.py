@@ -87,12 +87,27 @@ def test_linear_out_of_range_shard_gives_zero_columns():
 
 @pytest.mark.parametrize("K,M,slice_n", [(3, 9, 4096), (3, 300, 128), (4, 64, 192), (2, 33, 0), (6, 17, 256)])
 def test_linear_large_vs_oracle(K, M, slice_n):
-    """Above 8 rows: the input Hadamards, reconstructed fp16 weight slices (slice_n columns, 0 = whole groups) times xh
-    of each shard group in the library GEMM, then the output Hadamard."""
+    """Above 8 rows (csrc/linear_rows.hip), within the oracle's rounding points of the library-GEMM path: fp16 products.
+    slice_n says nothing to these kernels (test_linear_library_gemm_vs_oracle has the calls that it cuts)."""
     print(f"case linear large K={K} M={M} slice={slice_n}", flush=True)
     ck = olin.checkpoint(200 + K, 384, [256, 384, 128], K)
     g = _group(ck)
     xf, x = _x(11 + M, M, 384, torch.bfloat16)
+    y = g(x, slice_n=slice_n)
+    torch.cuda.synchronize()
+    r = _rel(y.float().cpu().numpy(), _round(olin.linear(xf, ck, "large"), torch.bfloat16))
+    assert r < TOL, r
+
+
+@pytest.mark.parametrize("K,cb,M,slice_n", [(3, 2, 9, 4096), (3, 2, 65, 0), (4, 1, 33, 64), (6, 0, 17, 96), (2, 2, 130, 128)])
+def test_linear_library_gemm_vs_oracle(K, cb, M, slice_n):
+    """Above 8 rows with more shards than linear_rows takes (17; its limit is 16): the input Hadamards, reconstructed fp16
+    weight slices (slice_n columns, 0 = whole groups) times xh of each shard group in the library GEMM, then the output
+    Hadamard."""
+    print(f"case linear library gemm K={K} cb={cb} M={M} slice={slice_n}", flush=True)
+    ck = olin.checkpoint(800 + K + cb, 256, [128] * 16 + [256], K, cb)
+    g = _group(ck)
+    xf, x = _x(21 + M, M, 256, torch.bfloat16)
     y = g(x, slice_n=slice_n)
     torch.cuda.synchronize()
     r = _rel(y.float().cpu().numpy(), _round(olin.linear(xf, ck, "large"), torch.bfloat16))
@@ -237,7 +252,7 @@ def test_linear_small_two_graphs_on_one_capture_stream():
 @pytest.mark.parametrize("cb", [0, 1])
 def test_codebooks_3inst_mcg_vs_oracle(K, cb):
     """The 3inst (0) and mcg (1) codebooks at K = 4 and 6: reconstructed weights bit-exact, the fused path at 1, 3 and
-    8 rows over one K-slice (k = 512) and over four (k = 2048, the tagged hand-off), and the large-M path, against the
+    8 rows over one K-slice (k = 512) and over four (k = 2048, the tagged hand-off), and the path above 8 rows, against the
     oracle."""
     from exl3xpu.linear import C
     print(f"case codebook cb={cb} K={K}", flush=True)

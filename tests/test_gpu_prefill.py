@@ -157,8 +157,8 @@ def test_prefill_large_expert_shapes(K):
 
 
 def test_prefill_full_chunk_vs_decode():
-    """8,192 tokens x 512 experts (H 2048, I 512, K=3), top-10: the prefill output against the decode kernel run on
-    64-row slices of the same inputs (fp32 activations and outputs: the only difference is the prefill's fp16 y), and
+    """8,192 tokens x 512 experts (H 2048, I 512, K=3), top-10: the prefill output against the fused decode kernel run
+    on 8-row slices of the same inputs (80 picks: below the sizes that the grouped kernels take; fp32 activations and outputs: the only difference is the prefill's fp16 y), and
     32 seeded rows of it against the oracle's prefill rounding points (expert_pair, variant "prefill")."""
     H, I, K, E, M, topk = 2048, 512, 3, 512, 8192, 10
     print("case prefill full chunk vs decode", flush=True)
@@ -183,8 +183,8 @@ def test_prefill_full_chunk_vs_decode():
     xs = torch.from_numpy(exl3.bf16_to_f32(x)).cuda()
     it, wt = torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda()
     dec = []
-    for m0 in range(0, M, 64):
-        dec.append(_ops().moe_forward(xs[m0:m0 + 64], it[m0:m0 + 64].contiguous(), wt[m0:m0 + 64].contiguous(),
+    for m0 in range(0, M, 8):
+        dec.append(_ops().moe_forward(xs[m0:m0 + 8], it[m0:m0 + 8].contiguous(), wt[m0:m0 + 8].contiguous(),
                                       table, I, K, E))
     torch.cuda.synchronize()
     dc = torch.cat(dec).cpu().numpy()
