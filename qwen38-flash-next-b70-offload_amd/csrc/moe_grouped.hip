@@ -305,10 +305,17 @@ static bool grouped_scales(size_t np, int E, bool host) { return np > (size_t)(h
 static size_t list_bytes(size_t n) { return align256((4 * n + 2) * 4); }
 static size_t big_items(size_t np) { return np / 65; }           // (an expert of more than 64 rows has 65 or more per item)
 
+// y starts 1 KiB into a page of 4 KiB: the combine reads the picks' rows and writes the output's at once, and with both on
+// page boundaries their lines fall on the same channels (8,192 tokens, H 2048: starts 0 / 256 / 512 / 1,024 / 2,048 / 3,072
+// bytes into a page 77 / 72 / 67 / 63 / 75 / 63 us)
+constexpr size_t kYPage = 4096;
+static uint8_t* y_start(uint8_t* p) { return p + ((1024 - (uintptr_t)p) & (kYPage - 1)); }
+
 size_t grouped_workspace_bytes(int M, int topk, int H, int I, int E, bool y32) {
     const size_t np = (size_t)pass_rows(M, topk, H, I) * topk;
-    return list_bytes(grouped_max_items(np, E)) + (y32 ? 0 : list_bytes(big_items(np))) + align256(np * 4) + align256(np * 4 * H) + align256(np * 2 * I) +
-           align256(np * H * (y32 ? 4 : 2)) + align256(std::min<size_t>(E, np / (y32 ? 16 : 2)) * 4 * H);
+    return list_bytes(grouped_max_items(np, E)) + (y32 ? 0 : list_bytes(big_items(np))) + align256(np * 4) +
+           align256(np * 4 * H) + align256(np * 2 * I) + align256(np * H * (y32 ? 4 : 2) + kYPage) +
+           align256(std::min<size_t>(E, np / (y32 ? 16 : 2)) * 4 * H);
 }
 
 static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) {
@@ -341,7 +348,7 @@ static hipError_t launch_pass(GroupedArgs a, bool y32, void* ws, hipStream_t s) 
     a.perm = (int*)take(np * 4);
     a.xh = (half_t*)take(np * 4 * a.g.H);
     a.abuf = (half_t*)take(np * 2 * a.g.I);
-    a.y = take(np * a.g.H * (y32 ? 4 : 2));
+    a.y = y_start(take(np * a.g.H * (y32 ? 4 : 2) + kYPage));
     a.suh = nullptr;
     if (grouped_scales(np, a.E, host)) {
         a.suh = (half_t*)take((size_t)a.E * 4 * a.g.H);
