@@ -138,16 +138,16 @@ int exl3_moe_forward_cached(const void* x, int x_dtype, int64_t x_stride, int M,
                             int n_experts, void* out, int64_t out_stride, void* workspace, size_t workspace_bytes,
                             void* stream);
 
-/* The same call without any allocation (no reference counterpart: the reference always passes a workspace that
- * torch allocates, a8:1229-1261). For callers that cannot allocate device memory: code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc. The decode scratch (the blob pointer of every pick and the
- * cross-workgroup exchange words, or the grouped kernels' workspace) comes from two static device arrays of
- * EXL3_STATIC_SCRATCH_BYTES (and 64 KiB) per device, held until the process ends; their addresses are looked up on
- * the first call on a device and the exchange words cleared then (one fill kernel on `stream`). Limit: calls whose scratch exceeds the array (8 MiB: config-0 shapes up to 25 rows x
- * top-10, config-4 shapes up to 7 rows x top-8) and calls that would take the uncached path (M >= prefill_min_m, or
- * n_slots == 0) fail with EXL3_EUNSUPPORTED before anything is enqueued. Every call on one device shares the array
- * and it keeps the last call's contents: calls that overlap on one device (other streams) race; stream-ordered calls
- * are safe. Decisions and outputs are those of exl3_moe_forward_cached. */
+/* The same call without any allocation (no reference counterpart: the reference always passes a workspace that torch
+ * allocates, a8:1229-1261). For callers that cannot allocate device memory: code under HIP graph capture, tight serving
+ * loops, harnesses that forbid hipMalloc. The decode scratch (the blob pointer of every pick and the cross-workgroup
+ * exchange words, or the grouped kernels' workspace) comes from two static device arrays of EXL3_STATIC_SCRATCH_BYTES
+ * (and 64 KiB) per device, held until the process ends; their addresses are looked up on the first call on a device and
+ * the exchange words cleared then (one fill kernel on `stream`). Limit: calls whose scratch exceeds the array (8 MiB:
+ * config-0 shapes up to 25 rows x top-10, config-4 shapes up to 7 rows x top-8) and calls that would take the uncached
+ * path (M >= prefill_min_m, or n_slots == 0) fail with EXL3_EUNSUPPORTED before anything is enqueued. Every call on one
+ * device shares the array and it keeps the last call's contents: calls that overlap on one device (other streams) race;
+ * stream-ordered calls are safe. Decisions and outputs are those of exl3_moe_forward_cached. */
 #define EXL3_STATIC_SCRATCH_BYTES ((size_t)8 << 20)
 int exl3_moe_forward_cached_static(const void* x, int x_dtype, int64_t x_stride, int M, int H, int32_t* topk_ids,
                                    float* topk_w, int topk, int64_t* ptrs_all, int layer, int32_t* slot_of,
@@ -276,9 +276,10 @@ int exl3_linear_small(const void* x, int x_dtype, int64_t x_stride, int M, int k
 
 /* The same linear for any number of rows, with the input Hadamards, the trellis decode and the products in kernels of
  * its own (exl3_ops.sycl:651-757, the path above the fused rows). group_bounds: host [S + 1], shard g's columns
- * [group_bounds[g], group_bounds[g + 1]), multiples of width (256 or 128). S at most 16. The workspace (device, exl3_linear_rows_workspace bytes, no state between calls) holds the input
- * Hadamards and the partial sums; its size is 0 for sizes that the call refuses (k not a multiple of 128, n not of width).
- * EXL3_EUNSUPPORTED if S M k fp16 values or the trellis reach 2 GiB. */
+ * [group_bounds[g], group_bounds[g + 1]), multiples of width (256 or 128). S at most 16. The workspace (device,
+ * exl3_linear_rows_workspace bytes, no state between calls) holds the input Hadamards and the partial sums; its size is
+ * 0 for sizes that the call refuses (k not a multiple of 128, n not of width). EXL3_EUNSUPPORTED if S M k fp16 values or
+ * the trellis reach 2 GiB. */
 size_t exl3_linear_rows_workspace(int M, int k, int n, int S, int width);
 int exl3_linear_rows(const void* x, int x_dtype, int64_t x_stride, int M, int k, int n, const void* trellis, int K,
                      int cb, const void* suh, int S, const void* svh, const int64_t* group_bounds, int width, void* out,

@@ -212,7 +212,7 @@ hipError_t launch_align(const int32_t* ids, const float* w, int npairs, int topk
                         const AlignOut& o, hipStream_t s);
 size_t align_scratch_bytes(int npairs, int E);
 
-// grouped.hip: y32 keeps the picks' outputs in fp32 (the decode sizes), else fp16 (as the prefill kernels do)
+// moe_grouped.hip: y32 keeps the picks' outputs in fp32 (the decode sizes), else fp16 (the prefill sizes)
 // an upper bound of a call's items: every expert's last one, and one more per 64 picks (items are cut at 64 rows or more)
 static inline size_t grouped_max_items(size_t np, int E) { return (np < (size_t)E ? np : (size_t)E) + np / 64; }
 // gate/up and down at bitrate K (moe_products.cuh)

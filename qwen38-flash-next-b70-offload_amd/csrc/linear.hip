@@ -14,8 +14,9 @@
 // (all loads of a round in flight together; bounded, a timeout counted in the device status words), sums the P slices
 // in order, applies the output Hadamard x svh and clears the words it read, so the exchange area is zero between
 // calls and needs no counter or epoch. k <= 512 (one slice): one workgroup of 8 waves per 128-column block, no hand-off.
-// More rows: linear_rows.hip. Shards that are not whole 128-column blocks, above the fused rows: the input-Hadamard
-// kernel, fp16 W slices (lin_reconstruct_kernel) for a library GEMM, then the output kernel on its fp16 product.
+// More rows: linear_rows.hip. Above the fused rows, more than 16 shards, S k above 2^22, a trellis of 2 GiB, or column
+// bounds that are not multiples of 128: the input-Hadamard kernel, fp16 W slices (lin_reconstruct_kernel) for a library
+// GEMM, then the output kernel on its fp16 product.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

@@ -262,7 +262,8 @@ static bool use_prefill(int M, int topk) { return M >= g_cfg.prefill_min_m || ex
 // once per pick: they take every call of the prefill sizes, and the decode sizes from picks * I = 56,000 on (49,000 for
 // experts of I >= 1024). Below that the fused kernel's single launch is faster, or the experts' workgroups divide badly
 // over the CUs: at H 2048 / I 512, top-10, 54 us against 67 us for 8 rows of distinct experts (80 picks), but 79 against
-// 56 us for 12 Zipf rows; at H 4096 / I 1536, top-8, K 4, 97 against 109 us for 3 rows and 126 against 110 us for 4.
+// 56 us for 12 Zipf rows; at H 4096 / I 1536, top-8, K 4, 97 against 109 us for 3 rows and 126 against 110 us for 4
+// (the two shapes that were measured, K 2 to 4; others go by the work).
 // Cached calls cross at the same sizes, with hits only and with misses: H 2048 / I 512, 11 rows, 100 / 99 / 95 / 90 % of
 // the experts in slots 88 / 99 / 175 / 301 against 61 / 98 / 175-179 / 288-295 us; H 4096 / I 1536, K 2, 4 rows
 // 128 / 147 / 235 / 364 against 112 / 134 / 229-234 / 354-366, K 3 133 / 168 / 329 / 542 against 113 / 146 / 292-302 / 487-502.

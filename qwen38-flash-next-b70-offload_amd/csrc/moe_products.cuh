@@ -152,8 +152,8 @@ __device__ __forceinline__ void gateup_rows(const GroupedArgs& A, int a, int s0,
     float4_t acc[NB][2][2];
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[b][0][0] = acc[b][0][1] = acc[b][1][0] = acc[b][1][1] = float4_t{};
-    regb_lds_core<K, NB, WV, 2, false, 2, kMoeSd, kMoePf<NB>>(rw, B::lane_off(tiles_n, pj * (I / 16) + nb * 2 * WV + wc * 4), tiles_n, ra,
-                                          soff, H / 64, pj, lds, acc);
+    regb_lds_core<K, NB, WV, 2, false, 2, kMoeSd, kMoePf<NB>>(
+        rw, B::lane_off(tiles_n, pj * (I / 16) + nb * 2 * WV + wc * 4), tiles_n, ra, soff, H / 64, pj, lds, acc);
     // 16 rows per round through one of two tiles [16][gate 32 WV | up 32 WV]: 16 lanes per (row, 128 columns)
     const int un = threadIdx.x >> 4, rr = un & 15, cb = (un >> 4) * 128 + (l & 15) * 8, ci = nb * 32 * WV + cb;
     const half8_u hg = ld_half8(base + A.g.off_svh_g + 2 * ci);
@@ -288,8 +288,10 @@ __device__ __forceinline__ void down_item(const GroupedArgs& A, int a, int s0, i
 }
 
 // One launch per product (two launches, one per item size, left the chip idle behind the longest item of each: a batch
-// of 64 rows took 193 us in two, 132 us in one). !BIG (items of up to 4 blocks): 4 waves per SIMD; the items of several blocks come first, then
-// those of one. BIG (items of up to 12 blocks): 2 waves per SIMD, block counts below 9 rounded up to 4, 6 or 8.
+// of 64 rows took 193 us in two, 132 us in one). !BIG (items of up to 4 blocks): 4 waves per SIMD; the items of several
+// blocks come first, then those of one. BIG (items of up to 12 blocks): 2 waves per SIMD, block counts below 9 rounded up
+// to 4, 6 or 8. A kernel holds up to seven instantiations of the core, and its largest sets the registers of all: at 128 and
+// 256 VGPRs the compiler spills 4-10 of them at K = 3, 8-31 at K = 4 (most in the 4-wave gate/up).
 // FILL: the instantiations that copy (exl3_fill.cuh); the copy inside the others would cost them up to 3 % in registers.
 template <int K, int WV, bool BIG, bool FILL>
 __global__ void __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(BIG ? 2 : 4)))

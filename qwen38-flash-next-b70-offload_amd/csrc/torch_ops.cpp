@@ -377,11 +377,11 @@ void linear_q8(const at::Tensor& x2, const at::Tensor& trellis, const at::Tensor
     }
 }
 
-// exl3_linear (exl3_ops.sycl:651-757): M <= small_m_max (at most 8 rows here) -> the fused path; otherwise, with shards of
-// whole 128-column blocks, exl3_linear_rows, which decodes the trellis inside the product (111 -> 26 us at 40 rows and
-// 689 -> 557 us at 8,192 rows of 2048 -> 12,288 against the following); else the input Hadamards, per shard group the
-// reconstructed fp16 weights in slices of slice_n columns times xh[g] (a library GEMM, fp16 output), then the output
-// Hadamard
+// exl3_linear (exl3_ops.sycl:651-757): M <= small_m_max (at most 8 rows here) -> the fused path; otherwise, with at most 16
+// shards of whole 128-column blocks, S k up to 2^22 and a trellis below 2 GiB, exl3_linear_rows, which decodes the trellis
+// inside the product (111 -> 26 us at 40 rows and 689 -> 557 us at 8,192 rows of 2048 -> 12,288 against the following);
+// else the input Hadamards, per shard group the reconstructed fp16 weights in slices of slice_n columns times xh[g] (a
+// library GEMM, fp16 output), then the output Hadamard. slice_n is the library GEMM's alone.
 at::Tensor linear(at::Tensor x, at::Tensor trellis, at::Tensor suh, at::Tensor svh, at::Tensor shard_of_nb,
                   at::IntArrayRef group_bounds, int64_t K, int64_t cb, int64_t small_m_max, int64_t slice_n) {
     auto shape = x.sizes().vec();
